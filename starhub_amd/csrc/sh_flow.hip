@@ -67,47 +67,111 @@ __device__ __forceinline__ float4 texel4(const float4 *__restrict__ m, int W, in
     return (x >= 0 && y >= 0 && x < W && y < H) ? m[size_t(y) * W + x] : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-__global__ void k_node_motion_sum(const float4 *__restrict__ rgbd_prev, const float4 *__restrict__ rgbd,
-                                  const float2 *__restrict__ flow, const uint32_t *__restrict__ index_prev,
-                                  const uint16_t *__restrict__ surfel_knn, const float *__restrict__ surfel_spatial,
-                                  MotionParams mp, unsigned long long *__restrict__ sums)
+// Neighbouring pixels mostly name the same few nodes, so the sums of a 16x16
+// tile go through a small LDS table (open addressing by node id, each entry
+// kept four times so that the lanes of a wave that name one node spread over
+// four addresses) and one global atomic per distinct node and component
+// follows.  A pixel that finds no entry within kMotionProbes adds to global
+// memory itself.  Integer sums: the same bits either way.  Bound before by
+// the serial 64-bit atomics on each node's line (1279x717, 2047 nodes: 418 us
+// before, 34 us now; 320x240, 512 nodes: 48 and 4.5 us).
+constexpr int kMotionTile = 16;
+constexpr uint32_t kMotionSlots = 64; // entries of the table (a power of two)
+constexpr uint32_t kMotionReps = 4;
+constexpr uint32_t kMotionProbes = 8;
+constexpr uint32_t kNoNode = 0xffffffffu;
+static_assert(kMotionTile * kMotionTile == int(kMotionSlots * 4), "one thread per (entry, component) in the flush");
+
+__global__ __launch_bounds__(kMotionTile *kMotionTile) void k_node_motion_sum(
+    const float4 *__restrict__ rgbd_prev, const float4 *__restrict__ rgbd, const float2 *__restrict__ flow,
+    const uint32_t *__restrict__ index_prev, const uint16_t *__restrict__ surfel_knn,
+    const float *__restrict__ surfel_spatial, MotionParams mp, unsigned long long *__restrict__ sums)
 {
-    const int xp = blockIdx.x * blockDim.x + threadIdx.x, yp = blockIdx.y * blockDim.y + threadIdx.y;
-    if (xp >= mp.width || yp >= mp.height)
-        return;
-    const size_t pp = size_t(yp) * mp.width + xp;
-    const float2 of = flow[pp];
-    const float xf = float(xp) + of.x, yf = float(yp) + of.y;
-    // point sampling at a float coordinate: the texel floor(x), zero outside
-    const float4 c = texel4(rgbd, mp.width, mp.height, int(floorf(xf)), int(floorf(yf)));
-    const uint32_t s = index_prev[pp];
-    const float4 cp = rgbd_prev[pp];
-    if (s == 0xffffffffu || c.w == 0.f)
-        return;
-    if (s >= mp.num_surfels)
-        return; // not a surfel of this geometry: contributes nothing
-    const uint32_t node = surfel_knn[size_t(s) * mp.K];
-    if (node >= mp.num_nodes)
-        return;
-    const float wgt = surfel_spatial[size_t(s) * mp.K];
-    const float depth = 1.f / c.w, depth_prev = 1.f / cp.w;
-    const float vx = (xf - mp.cx) / mp.fx * depth, vy = (yf - mp.cy) / mp.fy * depth, vz = depth;
-    const float ux = (float(xp) - mp.cx) / mp.fx * depth_prev, uy = (float(yp) - mp.cy) / mp.fy * depth_prev;
-    float mx = vx - ux, my = vy - uy, mz = vz - depth_prev;
-    if (fabsf(mz) > 0.05f) // optical_flow_z_shift, node_graph_opticalflow.cu:10
-        return;
-    mx *= wgt;
-    my *= wgt;
-    mz *= wgt;
-    const float wx = (mp.r[0] * mx + mp.r[1] * my) + mp.r[2] * mz;
-    const float wy = (mp.r[3] * mx + mp.r[4] * my) + mp.r[5] * mz;
-    const float wz = (mp.r[6] * mx + mp.r[7] * my) + mp.r[8] * mz;
-    // exact integer sums (two's complement wraps identically in any order)
-    unsigned long long *o = sums + size_t(node) * 4;
-    atomicAdd(o + 0, static_cast<unsigned long long>(llrintf(wx * kFixScale)));
-    atomicAdd(o + 1, static_cast<unsigned long long>(llrintf(wy * kFixScale)));
-    atomicAdd(o + 2, static_cast<unsigned long long>(llrintf(wz * kFixScale)));
-    atomicAdd(o + 3, static_cast<unsigned long long>(llrintf(wgt * kFixScale)));
+    __shared__ uint32_t key[kMotionSlots];
+    __shared__ unsigned long long acc[kMotionSlots][4][kMotionReps];
+    const uint32_t tid = threadIdx.y * kMotionTile + threadIdx.x;
+    if (tid < kMotionSlots)
+        key[tid] = kNoNode;
+#pragma unroll
+    for (uint32_t r = 0; r < kMotionReps; ++r)
+        acc[tid >> 2][tid & 3u][r] = 0ull;
+    const int xp = blockIdx.x * kMotionTile + threadIdx.x, yp = blockIdx.y * kMotionTile + threadIdx.y;
+    uint32_t node = kNoNode;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (xp < mp.width && yp < mp.height)
+    {
+        const size_t pp = size_t(yp) * mp.width + xp;
+        const float2 of = flow[pp];
+        const float xf = float(xp) + of.x, yf = float(yp) + of.y;
+        // point sampling at a float coordinate: the texel floor(x), zero outside
+        const float4 c = texel4(rgbd, mp.width, mp.height, int(floorf(xf)), int(floorf(yf)));
+        const uint32_t s = index_prev[pp];
+        const float4 cp = rgbd_prev[pp];
+        // a surfel that is not of this geometry contributes nothing
+        if (s != 0xffffffffu && c.w != 0.f && s < mp.num_surfels)
+        {
+            const uint32_t n = surfel_knn[size_t(s) * mp.K];
+            const float wgt = surfel_spatial[size_t(s) * mp.K];
+            const float depth = 1.f / c.w, depth_prev = 1.f / cp.w;
+            const float vx = (xf - mp.cx) / mp.fx * depth, vy = (yf - mp.cy) / mp.fy * depth, vz = depth;
+            const float ux = (float(xp) - mp.cx) / mp.fx * depth_prev, uy = (float(yp) - mp.cy) / mp.fy * depth_prev;
+            float mx = vx - ux, my = vy - uy, mz = vz - depth_prev;
+            // optical_flow_z_shift, node_graph_opticalflow.cu:10
+            if (n < mp.num_nodes && !(fabsf(mz) > 0.05f))
+            {
+                node = n;
+                mx *= wgt;
+                my *= wgt;
+                mz *= wgt;
+                v[0] = (mp.r[0] * mx + mp.r[1] * my) + mp.r[2] * mz;
+                v[1] = (mp.r[3] * mx + mp.r[4] * my) + mp.r[5] * mz;
+                v[2] = (mp.r[6] * mx + mp.r[7] * my) + mp.r[8] * mz;
+                v[3] = wgt;
+            }
+        }
+    }
+    __syncthreads();
+    if (node != kNoNode)
+    {
+        // exact integer sums (two's complement wraps identically in any order)
+        unsigned long long q[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            q[c] = static_cast<unsigned long long>(llrintf(v[c] * kFixScale));
+        uint32_t h = (node * 2654435761u) >> 26, probe = 0;
+        static_assert(kMotionSlots == 64, "hash bits");
+        for (; probe < kMotionProbes; ++probe, h = (h + 1u) & (kMotionSlots - 1u))
+        {
+            const uint32_t k = atomicCAS(&key[h], kNoNode, node);
+            if (k == kNoNode || k == node)
+                break;
+        }
+        if (probe < kMotionProbes)
+        {
+            const uint32_t r = threadIdx.x & (kMotionReps - 1u);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                atomicAdd(&acc[h][c][r], q[c]);
+        }
+        else
+        {
+            unsigned long long *o = sums + size_t(node) * 4;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                atomicAdd(o + c, q[c]);
+        }
+    }
+    __syncthreads();
+    const uint32_t n = key[tid >> 2], c = tid & 3u;
+    if (n != kNoNode)
+    {
+        unsigned long long t = 0ull;
+#pragma unroll
+        for (uint32_t r = 0; r < kMotionReps; ++r)
+            t += acc[tid >> 2][c][r];
+        if (t)
+            atomicAdd(sums + size_t(n) * 4 + c, t);
+    }
 }
 
 __global__ void k_zero_u64(unsigned long long *__restrict__ p, uint32_t n)
@@ -198,7 +262,9 @@ hipError_t launch_node_motion(const float *rgbd_prev4, const float *rgbd4, const
     mp.num_surfels = num_surfels;
     mp.num_nodes = num_nodes;
     if (width > 0 && height > 0)
-        hipLaunchKernelGGL(k_node_motion_sum, dim3((width + 15) / 16, (height + 15) / 16), dim3(16, 16), 0, st,
+        hipLaunchKernelGGL(k_node_motion_sum,
+                           dim3((width + kMotionTile - 1) / kMotionTile, (height + kMotionTile - 1) / kMotionTile),
+                           dim3(kMotionTile, kMotionTile), 0, st,
                            reinterpret_cast<const float4 *>(rgbd_prev4), reinterpret_cast<const float4 *>(rgbd4),
                            reinterpret_cast<const float2 *>(flow2), index_prev, surfel_knn, surfel_spatial, mp, sums);
     hipLaunchKernelGGL(k_node_motion_mean, dim3((num_nodes + 255) / 256), dim3(256), 0, st, sums, num_nodes,
