@@ -30,8 +30,11 @@ constexpr int kMSpan = kMTile + 2 * kApron; // 22
 
 __device__ __forceinline__ bool zero_vertex(float x, float y, float z)
 {
-    // is_zero_vertex (vector_ops.hpp:122-126): compared with the double literal
-    return fabs(double(x)) < 1e-3 && fabs(double(y)) < 1e-3 && fabs(double(z)) < 1e-3;
+    // is_zero_vertex (vector_ops.hpp:122-126) compares with the double literal
+    // 1e-3; 1e-3f is the smallest float not below it, so the float test decides
+    // the same way for every float
+    static_assert(double(1e-3f) >= 1e-3 && 1e-3 > 0.0, "the float threshold lies above the double one");
+    return fabsf(x) < 1e-3f && fabsf(y) < 1e-3f && fabsf(z) < 1e-3f;
 }
 
 __device__ __forceinline__ float3 cross3(float3 a, float3 b)
@@ -182,65 +185,83 @@ __device__ float3 smallest_eigvec(const float cov[6])
     }
     if (ev.z - ev.y <= FLT_EPSILON)
         return null_vector(m, ev.x, chosen, third);
-    float3 e[3];
-    float mmax[3];
-    e[2] = null_vector(m, ev.z, mmax[2], third);
-    e[1] = null_vector(m, ev.y, mmax[1], third);
-    unsigned min_el = 2, max_el = 2;
-    min_el = mmax[1] <= mmax[min_el] ? 1u : min_el;
-    max_el = mmax[1] > mmax[max_el] ? 1u : max_el;
-    e[0] = null_vector(m, ev.x, mmax[0], third);
-    min_el = third <= mmax[min_el] ? 0u : min_el; // the third product, in every branch
-    max_el = third > mmax[max_el] ? 0u : max_el;
-    const unsigned mid_el = 3u - min_el - max_el;
-    e[min_el] = normalized3(cross3(e[(min_el + 1) % 3], e[(min_el + 2) % 3]));
-    e[mid_el] = normalized3(cross3(e[(mid_el + 1) % 3], e[(mid_el + 2) % 3]));
-    return e[0];
+    // the three null vectors with the lengths they were chosen by; those with
+    // the smallest and the middle length are remade from the other two, in
+    // that order (eigen33's bookkeeping, where the third length is the third
+    // cross product's).  Only the vector of ev.x is returned, so it is written
+    // out for that one: arrays indexed by the picks would live in LDS or
+    // scratch memory.
+    float m2, m1, m0;
+    const float3 e2 = null_vector(m, ev.z, m2, third);
+    const float3 e1 = null_vector(m, ev.y, m1, third);
+    int min_el = m1 <= m2 ? 1 : 2, max_el = m1 > m2 ? 1 : 2;
+    const float lo = m1 <= m2 ? m1 : m2, hi = m1 > m2 ? m1 : m2;
+    const float3 e0 = null_vector(m, ev.x, m0, third);
+    min_el = third <= lo ? 0 : min_el; // the third product, in every branch
+    max_el = third > hi ? 0 : max_el;
+    if (min_el == 0)
+        return normalized3(cross3(e1, e2));
+    if (min_el == 1 && max_el == 2)
+        return normalized3(cross3(normalized3(cross3(e2, e0)), e2));
+    if (min_el == 2 && max_el == 1)
+        return normalized3(cross3(e1, normalized3(cross3(e0, e1))));
+    return e0;
+}
+
+// A window point as the tiles hold it: w = 1, or all zeros where there is no
+// valid vertex (zero_vertex), tested once per texel instead of once per window
+// that holds it (85 times).  A zero adds nothing to the window sums, and
+// the covariance takes its difference as 0, so neither loop branches.
+// With the window's rows not unrolled and no array indexed at run time the
+// kernels hold 52 registers instead of 190 and keep eight waves a SIMD, not
+// two; they are bound by the window's arithmetic (1279x717: filter 64 -> 33 us,
+// normals 61 -> 31 us).
+__device__ __forceinline__ float4 window_point(float x, float y, float z)
+{
+    return zero_vertex(x, y, z) ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(x, y, z, 1.f);
 }
 
 // The 7x7 window normal around LDS cell (lx, ly) of a kMSpan-wide tile of
-// float4 vertices (w unused): centroid of the valid points of the 7x7
+// window points: centroid of the valid points of the 7x7
 // window, covariance over the 6x6 window [-3, +2]^2, smallest eigenvector
 // oriented against the centre.  false: at most 24 valid points.
 __device__ bool window_normal(const float4 *tile, int lx, int ly, float3 center, float3 &normal)
 {
-    float cx = 0.f, cy = 0.f, cz = 0.f;
-    int counter = 0;
+    float cx = 0.f, cy = 0.f, cz = 0.f, counter = 0.f;
+    // rows one at a time: unrolled over the window the loads of all 85 points
+    // are hoisted, and their registers leave two waves a SIMD
+#pragma unroll 1
     for (int dy = -kApron; dy <= kApron; ++dy)
 #pragma unroll
         for (int dx = -kApron; dx <= kApron; ++dx)
         {
             const float4 p = tile[(ly + dy) * kMSpan + lx + dx];
-            if (!zero_vertex(p.x, p.y, p.z))
-            {
-                cx += p.x;
-                cy += p.y;
-                cz += p.z;
-                ++counter;
-            }
+            cx += p.x;
+            cy += p.y;
+            cz += p.z;
+            counter += p.w; // at most 49: exact
         }
-    if (counter <= 24)
+    if (counter <= 24.f)
         return false;
-    const float inv = 1.f / float(counter);
+    const float inv = 1.f / counter;
     cx *= inv;
     cy *= inv;
     cz *= inv;
     float cov[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
     for (int dy = -kApron; dy < kApron; ++dy)
 #pragma unroll
         for (int dx = -kApron; dx < kApron; ++dx)
         {
             const float4 p = tile[(ly + dy) * kMSpan + lx + dx];
-            if (!zero_vertex(p.x, p.y, p.z))
-            {
-                const float ux = p.x - cx, uy = p.y - cy, uz = p.z - cz;
-                cov[0] += ux * ux;
-                cov[1] += ux * uy;
-                cov[2] += ux * uz;
-                cov[3] += uy * uy;
-                cov[4] += uy * uz;
-                cov[5] += uz * uz;
-            }
+            const bool in = p.w != 0.f;
+            const float ux = in ? p.x - cx : 0.f, uy = in ? p.y - cy : 0.f, uz = in ? p.z - cz : 0.f;
+            cov[0] += ux * ux;
+            cov[1] += ux * uy;
+            cov[2] += ux * uz;
+            cov[3] += uy * uy;
+            cov[4] += uy * uz;
+            cov[5] += uz * uz;
         }
     float3 n = smallest_eigvec(cov);
     if (dot3(n, center) >= 0.f)
@@ -264,7 +285,7 @@ __global__ __launch_bounds__(kMTile *kMTile) void k_filter_depth(const uint16_t 
         const int gx = x0 + i % kMSpan, gy = y0 + i / kMSpan;
         const uint32_t d = (gx >= 0 && gy >= 0 && gx < W && gy < H) ? raw[size_t(gy) * W + gx] : 0u;
         const float z = float(d) / 1000.f;
-        tile[i] = make_float4((float(gx) - cx_) * inv_fx * z, (float(gy) - cy_) * inv_fy * z, z, 0.f);
+        tile[i] = window_point((float(gx) - cx_) * inv_fx * z, (float(gy) - cy_) * inv_fy * z, z);
     }
     __syncthreads();
     const int x = blockIdx.x * kMTile + threadIdx.x, y = blockIdx.y * kMTile + threadIdx.y;
@@ -283,12 +304,9 @@ __global__ __launch_bounds__(kMTile *kMTile) void k_filter_depth(const uint16_t 
         const float4 c4 = tile[ly * kMSpan + lx];
         const float3 vc = make_float3(c4.x, c4.y, c4.z);
         float3 nc = make_float3(0.f, 0.f, 0.f);
-        if (!zero_vertex(vc.x, vc.y, vc.z))
-        {
-            float3 n;
-            if (window_normal(tile, lx, ly, vc, n))
-                nc = n;
-        }
+        float3 n;
+        if (c4.w != 0.f && window_normal(tile, lx, ly, vc, n))
+            nc = n;
         const float ci = 1e-6f + sqrtf(dot3(vc, vc));
         const float ni = 1e-6f + sqrtf(dot3(nc, nc));
         const float3 cd = make_float3(vc.x / ci, vc.y / ci, vc.z / ci);
@@ -327,8 +345,9 @@ __global__ __launch_bounds__(kMTile *kMTile) void k_normal_radius(const float4 *
     for (int i = tid; i < kMSpan * kMSpan; i += kMTile * kMTile)
     {
         const int gx = x0 + i % kMSpan, gy = y0 + i / kMSpan;
-        tile[i] = (gx >= 0 && gy >= 0 && gx < w && gy < h) ? vertex[size_t(gy) * w + gx]
-                                                          : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 v = (gx >= 0 && gy >= 0 && gx < w && gy < h) ? vertex[size_t(gy) * w + gx]
+                                                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+        tile[i] = window_point(v.x, v.y, v.z);
     }
     __syncthreads();
     const int x = blockIdx.x * kMTile + threadIdx.x, y = blockIdx.y * kMTile + threadIdx.y;
@@ -338,7 +357,7 @@ __global__ __launch_bounds__(kMTile *kMTile) void k_normal_radius(const float4 *
     const float4 c4 = tile[ly * kMSpan + lx];
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     float3 n;
-    if (!zero_vertex(c4.x, c4.y, c4.z) && window_normal(tile, lx, ly, make_float3(c4.x, c4.y, c4.z), n))
+    if (c4.w != 0.f && window_normal(tile, lx, ly, make_float3(c4.x, c4.y, c4.z), n))
     {
         // compute_radius (normal_map.cu:9-22), [mm]
         const float radius = c4.z * (1000 * 1.414f / 570.0f) * radius_scale;
