@@ -1226,228 +1226,6 @@ __global__ void k_identity_dq(float4 *__restrict__ dq, uint32_t n_nodes)
     dq[2 * n + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// ============================================================ input producers
-// KNN heap: replace the current maximum, then a Lomuto quicksort ascending
-// (libs/star/geometry/node_graph/brute_force_knn.cuh:52-135).
-template <int K>
-struct KnnHeap
-{
-    float dist[K];
-    uint16_t idx[K];
-    int max_id;
-    float max_d;
-    __device__ void init(float d0)
-    {
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-        {
-            dist[k] = d0;
-            idx[k] = 0;
-        }
-        refresh();
-    }
-    __device__ __forceinline__ void refresh()
-    {
-        max_id = 0;
-        max_d = dist[0];
-#pragma unroll
-        for (int k = 1; k < K; ++k)
-            if (dist[k] > max_d)
-            {
-                max_d = dist[k];
-                max_id = k;
-            }
-    }
-    __device__ __forceinline__ void update(uint16_t id, float d)
-    {
-        if (d < max_d)
-        {
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-                if (k == max_id)
-                {
-                    dist[k] = d;
-                    idx[k] = id;
-                }
-            refresh();
-        }
-    }
-    // iterative Lomuto quicksort with the recursion order of the reference
-    __device__ void sort()
-    {
-        float dd[K];
-        uint16_t ii[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-        {
-            dd[k] = dist[k];
-            ii[k] = idx[k];
-        }
-        int stack_lo[2 * K], stack_hi[2 * K];
-        int top = 0;
-        stack_lo[0] = 0;
-        stack_hi[0] = K - 1;
-        top = 1;
-        while (top > 0)
-        {
-            --top;
-            const int lo = stack_lo[top], hi = stack_hi[top];
-            if (lo >= hi)
-                continue;
-            const float pivot = dd[hi];
-            int i = lo - 1;
-            for (int j = lo; j <= hi - 1; ++j)
-                if (dd[j] < pivot)
-                {
-                    ++i;
-                    const float tf = dd[i];
-                    dd[i] = dd[j];
-                    dd[j] = tf;
-                    const uint16_t ti = ii[i];
-                    ii[i] = ii[j];
-                    ii[j] = ti;
-                }
-            {
-                const float tf = dd[i + 1];
-                dd[i + 1] = dd[hi];
-                dd[hi] = tf;
-                const uint16_t ti = ii[i + 1];
-                ii[i + 1] = ii[hi];
-                ii[hi] = ti;
-            }
-            const int pi = i + 1;
-            // recursion order: left part first, then right part
-            stack_lo[top] = pi + 1;
-            stack_hi[top] = hi;
-            ++top;
-            stack_lo[top] = lo;
-            stack_hi[top] = pi - 1;
-            ++top;
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-        {
-            dist[k] = dd[k];
-            idx[k] = ii[k];
-        }
-    }
-};
-
-// fma(dz,dz,fma(dy,dy,dx*dx)) with no further contraction (NodeGraph.cu:32-34)
-__device__ __forceinline__ float sqdist_fma(float dx, float dy, float dz)
-{
-    return __fmaf_rn(dz, dz, __fmaf_rn(dy, dy, __fmul_rn(dx, dx)));
-}
-
-constexpr int kSkinTile = 256;
-
-// SkinnerKernel (Skinner.cu:10-94): nodes staged through LDS in tiles.
-template <int K>
-__global__ __launch_bounds__(256) void k_skin(const float4 *__restrict__ surfels, uint32_t S,
-                                              const float4 *__restrict__ nodes, uint32_t N, float r2,
-                                              uint16_t *__restrict__ knn, float *__restrict__ spatial,
-                                              float *__restrict__ connect)
-{
-    __shared__ float4 tile[kSkinTile];
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = s < S;
-    const float4 v = live ? surfels[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-    KnnHeap<K> h;
-    h.init(1e6f);
-    for (uint32_t base = 0; base < N; base += kSkinTile)
-    {
-        __syncthreads();
-        if (base + threadIdx.x < N)
-            tile[threadIdx.x] = nodes[base + threadIdx.x];
-        __syncthreads();
-        const uint32_t cnt = min(uint32_t(kSkinTile), N - base);
-        for (uint32_t i = 0; i < cnt; ++i)
-        {
-            const float4 nd = tile[i];
-            const float dd = sqdist_fma(__fsub_rn(v.x, nd.x), __fsub_rn(v.y, nd.y), __fsub_rn(v.z, nd.z));
-            h.update(uint16_t(base + i), dd);
-        }
-    }
-    if (!live)
-        return;
-    h.sort();
-    float w[K];
-    float wsum = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-    {
-        const float4 nd = nodes[h.idx[k]];
-        const float dd = sqdist_fma(__fsub_rn(v.x, nd.x), __fsub_rn(v.y, nd.y), __fsub_rn(v.z, nd.z));
-        w[k] = __expf(-dd / (2.f * r2));
-        wsum += w[k];
-    }
-    const float inv = 1.f / wsum;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-    {
-        knn[size_t(s) * K + k] = h.idx[k];
-        spatial[size_t(s) * K + k] = inv * w[k];
-        connect[size_t(s) * K + k] = 1.f;
-    }
-}
-
-// UpdateNodeDistanceKernel + BuildNodeGraphKernel + BuildNodeGraphPairKernel
-// + ResetNodeConnectionKernel (NodeGraph.cu:10-145): the FP16 distance of each
-// pair is recomputed on the fly instead of being stored as an N x N matrix.
-template <int K>
-__global__ __launch_bounds__(256) void k_node_graph(const float4 *__restrict__ nodes, uint32_t N, float r2,
-                                                    uint16_t *__restrict__ node_knn, float *__restrict__ node_spatial,
-                                                    uint16_t *__restrict__ edges, float *__restrict__ node_connect)
-{
-    __shared__ float4 tile[kSkinTile];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = i < N;
-    const float4 vi = live ? nodes[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    KnnHeap<K> h;
-    h.init(1e3f);
-    for (uint32_t base = 0; base < N; base += kSkinTile)
-    {
-        __syncthreads();
-        if (base + threadIdx.x < N)
-            tile[threadIdx.x] = nodes[base + threadIdx.x];
-        __syncthreads();
-        const uint32_t cnt = min(uint32_t(kSkinTile), N - base);
-        for (uint32_t jj = 0; jj < cnt; ++jj)
-        {
-            const uint32_t j = base + jj;
-            const float4 vj = tile[jj];
-            // distance is written for idx >= idy with v1 = node[idx], v2 = node[idy]
-            const float4 hi = (i >= j) ? vi : vj;
-            const float4 lo = (i >= j) ? vj : vi;
-            const float dd = sqdist_fma(__fsub_rn(hi.x, lo.x), __fsub_rn(hi.y, lo.y), __fsub_rn(hi.z, lo.z));
-            h.update(uint16_t(j), __half2float(__float2half_rn(dd)));
-        }
-    }
-    if (!live)
-        return;
-    h.sort();
-    float w[K];
-    float wsum = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-    {
-        w[k] = __expf(-h.dist[k] / (2.f * r2));
-        wsum += w[k];
-    }
-    const float inv = 1.f / wsum;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-    {
-        node_knn[size_t(i) * K + k] = h.idx[k];
-        node_spatial[size_t(i) * K + k] = w[k] * inv;
-        node_connect[size_t(i) * K + k] = 1.f;
-        const size_t e = size_t(i) * K + k;
-        edges[3 * e] = uint16_t(i);
-        edges[3 * e + 1] = h.idx[k];
-        edges[3 * e + 2] = uint16_t(k);
-    }
-}
-
 // ============================================================ host launchers
 #define SH_GRID(n, b) dim3(unsigned(((n) + (b)-1) / (b)))
 
@@ -1751,32 +1529,6 @@ hipError_t launch_update(const SolveDesc *sds, const uint32_t *wmap, int n_solve
                          hipStream_t st)
 {
     hipLaunchKernelGGL(k_update, dim3(n_wg), dim3(256), 0, st, sds, wmap, n_solve, parity);
-    return hipGetLastError();
-}
-
-hipError_t launch_skin(uint32_t K, const float4 *surfels, uint32_t S, const float4 *nodes, uint32_t N, float r2,
-                       uint16_t *knn, float *spatial, float *connect, hipStream_t st)
-{
-    if (S == 0)
-        return hipSuccess;
-    if (K == 8)
-        hipLaunchKernelGGL(k_skin<8>, SH_GRID(S, 256), dim3(256), 0, st, surfels, S, nodes, N, r2, knn, spatial,
-                           connect);
-    else
-        hipLaunchKernelGGL(k_skin<4>, SH_GRID(S, 256), dim3(256), 0, st, surfels, S, nodes, N, r2, knn, spatial,
-                           connect);
-    return hipGetLastError();
-}
-
-hipError_t launch_node_graph(uint32_t K, const float4 *nodes, uint32_t N, float r2, uint16_t *node_knn,
-                             float *node_spatial, uint16_t *edges, float *node_connect, hipStream_t st)
-{
-    if (K == 8)
-        hipLaunchKernelGGL(k_node_graph<8>, SH_GRID(N, 256), dim3(256), 0, st, nodes, N, r2, node_knn, node_spatial,
-                           edges, node_connect);
-    else
-        hipLaunchKernelGGL(k_node_graph<4>, SH_GRID(N, 256), dim3(256), 0, st, nodes, N, r2, node_knn, node_spatial,
-                           edges, node_connect);
     return hipGetLastError();
 }
 
