@@ -102,6 +102,31 @@ struct SolveDesc
     float *mf_reg;    // E*3 per-edge J x
 };
 
+// The item of a work map that work-group wg belongs to: the last i < n with
+// begin[i] <= wg.  Up to 64 items are looked at at once, one per lane (the
+// binary search is a chain of dependent loads at the head of every batched
+// kernel).  Every lane of the calling wave must be active.
+__device__ __forceinline__ int find_item(const uint32_t *__restrict__ begin, int n, uint32_t wg)
+{
+    if (n == 1)
+        return 0;
+    if (n <= 64)
+    {
+        const int lane = int(threadIdx.x & 63u);
+        return __popcll(__ballot(lane < n && begin[lane < n ? lane : 0] <= wg)) - 1;
+    }
+    int lo = 0, hi = n;
+    while (hi - lo > 1)
+    {
+        const int mid = (lo + hi) >> 1;
+        if (begin[mid] <= wg)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
 // A generic pointer that is known to name device (global) memory.  The pointers
 // a kernel reads out of a descriptor array are generic, so their accesses
 // compile to flat_* instructions, which count against the LDS counter as well:

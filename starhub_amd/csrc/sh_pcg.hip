@@ -25,20 +25,6 @@ constexpr int kCoopThreads = 512;
 constexpr int kCoopWaves = kCoopThreads / 64;
 constexpr unsigned kSpinCap = 1u << 22; // default polls per barrier wait
 
-__device__ __forceinline__ int find_solve_p(const uint32_t *__restrict__ begin, int n, uint32_t wg)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (begin[mid] <= wg)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // First row whose first block is at or after block index t (rows are whole).
 __device__ __forceinline__ uint32_t row_at_block(const uint32_t *__restrict__ row_ptr, uint32_t n, uint32_t t)
 {
@@ -140,7 +126,7 @@ __global__ __launch_bounds__(kCoopThreads) void k_pcg_coop(const SolveDesc *__re
 {
     extern __shared__ float qblk[]; // tile x 6
     __shared__ double sh[kCoopWaves + 1];
-    const int si = find_solve_p(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t b0 = wg_begin[si], G = wg_begin[si + 1] - b0, g = blockIdx.x - b0;
     const uint32_t N = uint32_t(d.N);
@@ -320,7 +306,7 @@ __global__ __launch_bounds__(kResThreads) void k_pcg_resident(const SolveDesc *_
     __shared__ float qblk[kResThreads * kResBlocksPerThread * 6];
     __shared__ float rsh[kResThreads];
     __shared__ double sh[kCoopWaves + 1];
-    const int si = find_solve_p(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t b0 = wg_begin[si], G = wg_begin[si + 1] - b0, g = blockIdx.x - b0;
     const uint32_t N = uint32_t(d.N);
@@ -619,7 +605,7 @@ __global__ __launch_bounds__(kResThreads) void k_pcg_pipe(const SolveDesc *__res
     // a launch may cover a subset of the solves (wg_begin points into the
     // whole batch's map): its groups are numbered from wg_begin[0]
     const uint32_t bid = blockIdx.x + wg_begin[0];
-    const int si = find_solve_p(wg_begin, n_solve, bid);
+    const int si = find_item(wg_begin, n_solve, bid);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t b0 = wg_begin[si], G = wg_begin[si + 1] - b0, g = bid - b0;
     const uint32_t N = uint32_t(d.N);
@@ -893,7 +879,7 @@ __global__ __launch_bounds__(kResThreads) void k_pcg_pipe(const SolveDesc *__res
         // (k_update's work, with its cost reduction on each solve's group 0)
         rsh[tid] = own ? double(float(x)) : 0.0;
         __syncthreads();
-        if (g == 0 && tid < 64)
+        if (g == 0 && tid >= kResThreads - 64) // a wave that holds no node (at most 85 a group)
             reduce_cost(d, d.gn_iter + update_parity);
         if (tid < r1 - r0)
         {

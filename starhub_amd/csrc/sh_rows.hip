@@ -17,20 +17,6 @@
 
 namespace sh
 {
-__device__ __forceinline__ int find_solve_r(const uint32_t *__restrict__ begin, int n, uint32_t wg)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (begin[mid] <= wg)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 constexpr int kRowThreads = 256;
 
 // Entry (c, q) of the x-side ARAP row [-[p]x, I]:  q < 3 -> -skew(p)[c][q],
@@ -63,7 +49,7 @@ __global__ __launch_bounds__(kRowThreads) void k_row_bitmap(IndexGroup g, const 
     constexpr int kNodes = kRowThreads / TPN;
     __shared__ uint32_t bits_all[kNodes][kMaxWords];
     __shared__ uint32_t cnt[kNodes][2];
-    const int it = find_solve_r(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t slot = threadIdx.x / TPN, lane = threadIdx.x % TPN;
@@ -192,7 +178,7 @@ __global__ __launch_bounds__(kRowThreads) void k_row_cols(IndexGroup g, const ui
                                                           int cols)
 {
     static_assert(kMaxWords == 128 && kRowThreads == 64 * kRowNodes, "two bitmap words a lane, a wave per node");
-    const int it = find_solve_r(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t lane = threadIdx.x & 63u;
@@ -285,7 +271,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_seg(const SolveDesc *__res
                                                           uint32_t chunk)
 {
     extern __shared__ float smem[];
-    const int si = find_solve_r(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t seg = blockIdx.x - wg_begin[si];
     if (seg >= uint32_t(d.n_seg))
@@ -443,7 +429,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_combine(const SolveDesc *_
                                                               const uint32_t *__restrict__ wg_begin, int n_solve)
 {
     extern __shared__ float smem[];
-    const int si = find_solve_r(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t i = blockIdx.x - wg_begin[si];
     if (i >= uint32_t(d.N))

@@ -66,20 +66,6 @@ struct TileGeom
     static_assert(kPairs % 2 == 0 && TP <= int(kTilePixMax), "tile geometry");
 };
 
-__device__ __forceinline__ int find_solve_t(const uint32_t *__restrict__ begin, int n, uint32_t wg)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (begin[mid] <= wg)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // Full-block index of (lo, hi): the diagonal block of row lo for lo == hi,
 // else the position of hi among row lo's ascending neighbours, base + 1 + the
 // neighbours below hi, counted from row lo's bitmap word that holds hi and
@@ -228,7 +214,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
     } sm;
     __shared__ uint32_t last_key[G::kThreads];
     __shared__ uint32_t red[16];
-    const int it = find_solve_t(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t t = blockIdx.x - wmap[it], tid = threadIdx.x;
@@ -547,7 +533,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_compact(IndexGroup g, con
                                                                uint32_t *__restrict__ sort_vals)
 {
     using G = TileGeom<K, TP>;
-    const int it = find_solve_t(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t t = blockIdx.x - wmap[it], tid = threadIdx.x;
@@ -596,7 +582,7 @@ static_assert(kTileThreads == 64 * kRowNodes, "k_block_transpose: one wave per n
 __global__ __launch_bounds__(kTileThreads) void k_block_transpose(IndexGroup g, const uint32_t *__restrict__ wmap,
                                                                   IndexWs ws)
 {
-    const int it = find_solve_t(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint2 *__restrict__ bitpre = ws.bitpre + size_t(item.node0) * kBitmapWords;
@@ -641,7 +627,7 @@ __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ 
     extern __shared__ uint16_t slot_lds[];
     uint16_t *__restrict__ sst = slot_lds;
     uint16_t *__restrict__ perm = slot_lds + slot_cap + 2;
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t t = blockIdx.x - wg_begin[si];
     if (t >= uint32_t(d.n_tiles))
@@ -1234,7 +1220,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tiles_combine_wg(const SolveDe
     // has a work-group for every one of its groups)
     if (slots2 && blockIdx.x < n_slots2 && threadIdx.x < 4)
         slots2[blockIdx.x].v[threadIdx.x >> 1][threadIdx.x & 1] = 0.0;
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t i = blockIdx.x - wg_begin[si];
     if (i >= uint32_t(d.N))
@@ -1451,7 +1437,7 @@ __global__ __launch_bounds__(64) void k_tiles_combine_wave(const SolveDesc *__re
     // has a work-group for every one of its groups)
     if (slots2 && blockIdx.x < n_slots2 && threadIdx.x < 4)
         slots2[blockIdx.x].v[threadIdx.x >> 1][threadIdx.x & 1] = 0.0;
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t i = blockIdx.x - wg_begin[si];
     if (i >= uint32_t(d.N))
@@ -1656,7 +1642,7 @@ __global__ __launch_bounds__(2 * TP) void k_mf_tiles(const SolveDesc *__restrict
     __shared__ float wS[TP * K];
     __shared__ uint16_t ent[G::kEnt];
     __shared__ uint16_t sst[G::kEnt + 1];
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t t = blockIdx.x - wg_begin[si];
     if (t >= uint32_t(d.n_tiles))
@@ -1743,7 +1729,7 @@ __global__ __launch_bounds__(64) void k_mf_rows(const SolveDesc *__restrict__ sd
                                                 const uint32_t *__restrict__ wg_begin, int n_solve, int k_it,
                                                 const float *__restrict__ x_user, float *__restrict__ y_user)
 {
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t i = blockIdx.x - wg_begin[si];
     if (i >= uint32_t(d.N))
@@ -1858,7 +1844,7 @@ __global__ __launch_bounds__(64) void k_spmv_rows(const SolveDesc *__restrict__ 
                                                   const uint32_t *__restrict__ wg_begin, int n_solve,
                                                   const float *__restrict__ x, float *__restrict__ y)
 {
-    const int si = find_solve_t(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t i = blockIdx.x - wg_begin[si];
     if (i >= uint32_t(d.N))
@@ -2030,7 +2016,7 @@ __global__ __launch_bounds__(256) void k_slot_lists(IndexGroup g, const uint32_t
                                                     const uint32_t *__restrict__ skeys,
                                                     const uint32_t *__restrict__ svals)
 {
-    const int it = find_solve_t(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t S = d.tile_sbase[d.n_tiles];

@@ -20,9 +20,20 @@ __device__ __forceinline__ dq8 load_dq(const dq8 *__restrict__ a, uint32_t i)
 __device__ inline void reduce_cost(const SolveDesc &d, int slot)
 {
     const uint32_t n = (uint32_t(d.P) + 63u) / 64u + (uint32_t(d.E + d.N) + 255u) / 256u;
+    // eight loads in flight: one by one the sum of a large frame's partials is
+    // a chain of memory latencies (1280x720: about 3,800 partials, 60 a lane)
+    constexpr uint32_t kU = 8;
     double v = 0.0;
-    for (uint32_t i = threadIdx.x % 64u; i < n; i += 64)
-        v += d.cost_part[i];
+    for (uint32_t i0 = threadIdx.x % 64u; i0 < n; i0 += 64 * kU)
+    {
+        double c[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            c[u] = i0 + 64 * u < n ? d.cost_part[i0 + 64 * u] : 0.0;
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            v += c[u];
+    }
     v = wave_sum(v);
     if (threadIdx.x % 64u == 0)
         d.cost[slot] = v;
