@@ -218,7 +218,7 @@ int Engine::init(const sh_solver_config &c, uint32_t max_slots)
     d_wmaps_ = static_cast<char *>(d_descs_) + size_t(max_slots) * sizeof(SolveDesc);
     const size_t pcg_wg = size_t(max_slots) * div_up(ncap_, kPcgNodesPerWg);
     A(d_part_rs_, pcg_wg * 8);
-    A(d_part_dq_, pcg_wg * 8);
+    A(d_part_dq_, pcg_wg * kPcgSpmvPer * 8);
     A(d_slots_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot));
     A(d_slots2_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot2));
     A(d_flags_, 64);
@@ -1179,7 +1179,8 @@ hipError_t Engine::enqueue_pcg_launches(uint32_t ns, bool matrix_free, hipStream
         }
         else
             SH_TRY(launch_pcg_spmv(sds, map(kMapPcg, ns), n, map_total_[kMapPcg], int(k), prs, pdq, st));
-        SH_TRY(launch_pcg_update(sds, map(kMapPcg, ns), n, map_total_[kMapPcg], int(k), pdq, prs, st));
+        SH_TRY(launch_pcg_update(sds, map(kMapPcg, ns), n, map_total_[kMapPcg], int(k), matrix_free ? 1u : kPcgSpmvPer,
+                                 pdq, prs, st));
     }
 #undef SH_TRY
     return hipSuccess;

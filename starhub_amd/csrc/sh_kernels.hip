@@ -14,20 +14,6 @@
 
 namespace sh
 {
-__device__ __forceinline__ int find_solve(const uint32_t *__restrict__ begin, int n, uint32_t wg)
-{
-    int lo = 0, hi = n;
-    while (hi - lo > 1)
-    {
-        const int mid = (lo + hi) >> 1;
-        if (begin[mid] <= wg)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 // __float2uint_rn with saturation, NaN -> 0 (ImageTermKNNFetcher.cu:164-165)
 __device__ __forceinline__ uint32_t f2u_rn_sat(float v)
 {
@@ -76,7 +62,7 @@ __device__ __forceinline__ uint32_t tile_order(uint32_t x, uint32_t y, uint32_t 
 __global__ __launch_bounds__(256) void k_pixel_flags(IndexGroup g, const uint32_t *__restrict__ wmap, bool tiled,
                                                      IndexWs ws)
 {
-    const int it = find_solve(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc &d = g.sds[item.slot];
     const uint32_t W = uint32_t(d.W), H = uint32_t(d.H), N = uint32_t(d.N), E = uint32_t(d.E);
@@ -150,7 +136,7 @@ __global__ __launch_bounds__(256) void k_compact_pixels(IndexGroup g, const uint
                                                         IndexWs ws, uint32_t *__restrict__ kv_keys,
                                                         uint32_t *__restrict__ kv_vals)
 {
-    const int it = find_solve(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t blk = blockIdx.x - wmap[it];
@@ -321,7 +307,7 @@ __global__ __launch_bounds__(256) void k_n2t_split(IndexGroup g, const uint32_t 
                                                    const uint32_t *__restrict__ skeys,
                                                    const uint32_t *__restrict__ svals)
 {
-    const int it = find_solve(wmap, g.n, blockIdx.x);
+    const int it = find_item(wmap, g.n, blockIdx.x);
     const IndexItem item = g.items[it];
     const SolveDesc d = global_desc(g.sds[item.slot]);
     const uint32_t N = uint32_t(d.N);
@@ -582,7 +568,7 @@ template <int K, class JT>
 __device__ __forceinline__ void dense_terms_wg(const SolveDesc *__restrict__ sds, const uint32_t *__restrict__ wg_begin,
                                                int n_solve, uint32_t wg, int parity, int store)
 {
-    const int si = find_solve(wg_begin, n_solve, wg);
+    const int si = find_item(wg_begin, n_solve, wg);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t p = (wg - wg_begin[si]) * blockDim.x + threadIdx.x;
     double pix_cost = 0.0;
@@ -601,7 +587,7 @@ __device__ __forceinline__ void dense_terms_wg(const SolveDesc *__restrict__ sds
 __device__ __forceinline__ void reg_terms_wg(const SolveDesc *__restrict__ sds, const uint32_t *__restrict__ wg_begin,
                                              int n_solve, uint32_t wg, int parity, int store)
 {
-    const int si = find_solve(wg_begin, n_solve, wg);
+    const int si = find_item(wg_begin, n_solve, wg);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t item = (wg - wg_begin[si]) * blockDim.x + threadIdx.x;
     const dq8 *__restrict__ dq = pick2(d.dq, (d.gn_iter + parity) & 1);
@@ -697,7 +683,7 @@ __global__ __launch_bounds__(256) void k_diag_rhs(const SolveDesc *__restrict__ 
                                                   const uint32_t *__restrict__ wg_begin, int n_solve)
 {
     __shared__ float stage[4][48];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t n = (blockIdx.x - wg_begin[si]) * 4 + wave;
@@ -825,7 +811,7 @@ __global__ __launch_bounds__(256) void k_dinv(const SolveDesc *__restrict__ sds,
 #pragma unroll
         for (int a = 0; a < 4; ++a)
             slots2[gid].v[a >> 1][a & 1] = 0.0;
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t n = (blockIdx.x - wg_begin[si]) * blockDim.x + threadIdx.x;
     if (n >= uint32_t(d.N))
@@ -859,7 +845,7 @@ __global__ __launch_bounds__(256) void k_offdiag(const SolveDesc *__restrict__ s
                                                  int n_solve)
 {
     __shared__ float stage[4][36];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t u = (blockIdx.x - wg_begin[si]) * 4 + wave;
@@ -942,15 +928,19 @@ __global__ __launch_bounds__(256) void k_offdiag(const SolveDesc *__restrict__ s
 }
 
 // ============================================================ PCG
-// Work-groups of 192 threads = 32 node blocks x 6 rows; one solve per group.
-constexpr int kPcgNodes = 32;
+// Work-groups of 192 threads = 32 node blocks x 6 rows (the SpMV:
+// work-groups of eight nodes); one solve per group.  The SpMV reads the
+// direction and the preconditioned residual of a node together, so the split
+// kernels keep them as pairs (d, s), by iteration parity, in the vectors that
+// the pipelined PCG exchanges (mv: the two never run at once on a solve).
+constexpr int kPcgNodes = kPcgNodesPerWg;
 constexpr int kPcgThreads = kPcgNodes * 6;
 
 __device__ __forceinline__ double block_sum_192(double v, double *sh)
 {
     v = wave_sum(v);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0)
+    if (lane == 0 && wave < kPcgThreads / 64)
         sh[wave] = v;
     __syncthreads();
     const double r = sh[0] + sh[1] + sh[2];
@@ -958,15 +948,38 @@ __device__ __forceinline__ double block_sum_192(double v, double *sh)
     return r;
 }
 
-// Sum of the per-group partials of one solve, fixed order, broadcast to the group.
+// Orders the LDS accesses of one wave's lanes.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sum of the per-group partials of one solve, fixed order, in every lane of a wave.
+__device__ __forceinline__ double reduce_partials_wave(const double *__restrict__ part, uint32_t b0, uint32_t b1)
+{
+    constexpr uint32_t kU = 4; // loads in flight
+    double v = 0.0;
+    for (uint32_t i0 = b0 + (threadIdx.x & 63u); i0 < b1; i0 += 64 * kU)
+    {
+        double c[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            c[u] = i0 + 64 * u < b1 ? part[i0 + 64 * u] : 0.0;
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            v += c[u];
+    }
+    return wave_sum(v);
+}
+
+// The same, broadcast to the group.
 __device__ __forceinline__ double reduce_partials(const double *__restrict__ part, uint32_t b0, uint32_t b1, double *sh)
 {
-    double v = 0.0;
     if (threadIdx.x < 64)
     {
-        for (uint32_t i = b0 + threadIdx.x; i < b1; i += 64)
-            v += part[i];
-        v = wave_sum(v);
+        const double v = reduce_partials_wave(part, b0, b1);
         if (threadIdx.x == 0)
             sh[3] = v;
     }
@@ -983,7 +996,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_init(const SolveDesc *__res
 {
     __shared__ double sh[4];
     __shared__ float rb[kPcgThreads];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t node = (blockIdx.x - wg_begin[si]) * kPcgNodes + threadIdx.x / 6;
     const int a = threadIdx.x % 6;
@@ -1006,6 +1019,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_init(const SolveDesc *__res
         d.s[row] = sf;
         d.x[row] = 0.f;
         d.dv[0][row] = 0.f;
+        reinterpret_cast<float2 *>(d.mv[0])[row] = make_float2(0.f, sf);
         prod = double(r) * double(sf);
     }
     const double tot = block_sum_192(prod, sh);
@@ -1021,76 +1035,116 @@ __device__ __forceinline__ float d_next(double beta, float dold, float s)
 // d_k = s + beta d_{k-1}, q = A d_k (materialised blocks), partial d.q
 // (performSparseMVKernel + blockPCGThirdUpdateKernel, BlockPCG.cuh:175-189,
 // BinBlockCSR.cuh:7-35).
-__global__ __launch_bounds__(kPcgThreads) void k_pcg_spmv(const SolveDesc *__restrict__ sds,
-                                                          const uint32_t *__restrict__ wg_begin, int n_solve, int k,
-                                                          const double *__restrict__ part_rs,
-                                                          double *__restrict__ part_dq)
+// One wave takes eight block rows, a lane a scalar row, and adds its products
+// in block and column order.  Each lane reads one (d_{k-1}, s) pair of a
+// block's column, forms d_k once and hands it to the row's six lanes through
+// LDS (a lane used to gather all twelve values and form six); kU blocks are in
+// flight and the next kU on the way, without branches among the loads.  The
+// launch is bound by that chain of loads (row, column, vector): twelve solves
+// of 128 to 4096 nodes took 18.5 us with 32 rows a work-group and now take
+// 13 us.  Measured and not taken: a work-group's blocks through LDS as float4s
+// (16 us: its barriers and LDS cost more than its wide loads give), three
+// teams of nine lanes a row with a float4 each (12 us, but another order of
+// the sums), two or four nodes a work-group (the partials' reduction grows).
+constexpr uint32_t kSpmvNodes = kPcgNodes / kPcgSpmvPer;
+__global__ __launch_bounds__(64, 2) void k_pcg_spmv(const SolveDesc *__restrict__ sds,
+                                                    const uint32_t *__restrict__ wg_begin, int n_solve, int k,
+                                                    const double *__restrict__ part_rs, double *__restrict__ part_dq)
 {
-    __shared__ double sh[4];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    constexpr uint32_t kU = 4; // blocks of a row in flight, and as many more on the way
+    __shared__ v2f xs[2][kU][kSpmvNodes * 3];
+    static_assert(kSpmvNodes * 6 <= 64, "the work-group's rows fit one wave");
+    const uint32_t wg = blockIdx.x / kPcgSpmvPer, lane = threadIdx.x;
+    const int si = find_item(wg_begin, n_solve, wg);
     const SolveDesc d = global_desc(sds[si]);
-    const double delta = reduce_partials(part_rs, wg_begin[si], wg_begin[si + 1], sh);
+    const uint32_t node = (blockIdx.x - wg_begin[si] * kPcgSpmvPer) * kSpmvNodes + lane / 6, a = lane % 6;
+    const bool own = lane < kSpmvNodes * 6 && node < uint32_t(d.N);
+    const uint32_t row = own ? node : 0u;
+    uint32_t b = d.row_ptr[row] + row;
+    const uint32_t b1 = d.row_ptr[row + 1] + row + 1, last = b1 - 1; // at least one block a row
+    const v2f *__restrict__ ds = reinterpret_cast<const v2f *>(pick2(d.mv, k & 1));
+    // past the row's end its last block again (not added): no branches among the loads
+    auto columns = [&](uint32_t c0, uint32_t (&col)[kU]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+            col[u] = d.blk_col[min(c0 + u, last)];
+    };
+    auto entries = [&](uint32_t c0, const uint32_t (&col)[kU], v2f (&av)[kU][3], v2f (&pv)[kU])
+                       __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
+        {
+            const v2f *A = reinterpret_cast<const v2f *>(d.blk + size_t(min(c0 + u, last)) * 36 + 6 * a); // 8-byte aligned
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                av[u][c] = A[c];
+            pv[u] = ds[size_t(col[u]) * 6 + a];
+        }
+    };
+    uint32_t col[kU], coln[kU];
+    v2f av[kU][3], pv[kU], an[kU][3], pn[kU];
+    columns(b, col);
+    columns(b + kU, coln);
+    entries(b, col, av, pv);
+    const double delta = reduce_partials_wave(part_rs, wg_begin[si], wg_begin[si + 1]);
     double beta = 0.0;
     if (k > 0 && d.delta[k - 1] != 0.0)
         beta = delta / d.delta[k - 1];
-    if (threadIdx.x == 0 && blockIdx.x == wg_begin[si])
+    if (lane == 0 && blockIdx.x == wg_begin[si] * kPcgSpmvPer)
         d.delta[k] = delta;
-    const float *__restrict__ dold = pick2(d.dv, k & 1);
-    float *__restrict__ dnew = pick2(d.dv, (k + 1) & 1);
-    const uint32_t node = (blockIdx.x - wg_begin[si]) * kPcgNodes + threadIdx.x / 6;
-    const int a = threadIdx.x % 6;
-    double prod = 0.0;
-    if (node < uint32_t(d.N))
+    float acc = 0.f;
+    const uint32_t n_rounds = own ? (b1 - b + kU - 1) / kU : 0u;
+    for (uint32_t r = 0; __any(r < n_rounds); ++r)
     {
-        const size_t row = size_t(node) * 6 + a;
-        const float dn = d_next(beta, dold[row], d.s[row]);
-        dnew[row] = dn;
-        const uint32_t b0 = d.row_ptr[node] + node;
-        const uint32_t b1 = d.row_ptr[node + 1] + node + 1;
-        float acc = 0.f;
-        // four blocks per round: their loads are issued before their products,
-        // which are summed in block order (the same sums as one block a round)
-        constexpr int kU = 4;
-        uint32_t bb = b0;
-        for (; bb + kU <= b1; bb += kU)
+        if (__any(r + 1 < n_rounds))
         {
-            uint32_t col[kU];
+            entries(b + kU, coln, an, pn);
+            columns(b + 2 * kU, coln);
+        }
+        float *__restrict__ x = reinterpret_cast<float *>(&xs[r & 1][0][0]);
+        if (lane < kSpmvNodes * 6)
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
-                col[u] = d.blk_col[bb + u];
-            float av[kU][6], xv[kU][6];
+            for (uint32_t u = 0; u < kU; ++u)
+                x[u * kSpmvNodes * 6 + lane] = d_next(beta, pv[u].x, pv[u].y);
+        wave_lds_order();
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
+        for (uint32_t u = 0; u < kU; ++u)
+        {
+            const v2f *xr = &xs[r & 1][u][min(lane / 6, kSpmvNodes - 1u) * 3];
+            float t = acc;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
             {
-                const float *A = d.blk + size_t(bb + u) * 36 + 6 * a;
-                const size_t cr = size_t(col[u]) * 6;
-#pragma unroll
-                for (int c = 0; c < 6; ++c)
-                {
-                    av[u][c] = A[c];
-                    xv[u][c] = d_next(beta, dold[cr + c], d.s[cr + c]);
-                }
+                const v2f v = xr[c];
+                t += av[u][c].x * v.x;
+                t += av[u][c].y * v.y;
             }
-#pragma unroll
-            for (int u = 0; u < kU; ++u)
-#pragma unroll
-                for (int c = 0; c < 6; ++c)
-                    acc += av[u][c] * xv[u][c];
+            acc = own && b + u < b1 ? t : acc;
         }
-        for (; bb < b1; ++bb)
+        b += kU;
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u)
         {
-            const uint32_t col = d.blk_col[bb];
-            const float *A = d.blk + size_t(bb) * 36 + 6 * a;
-            const size_t cr = size_t(col) * 6;
+            pv[u] = pn[u];
 #pragma unroll
-            for (int c = 0; c < 6; ++c)
-                acc += A[c] * d_next(beta, dold[cr + c], d.s[cr + c]);
+            for (int c = 0; c < 3; ++c)
+                av[u][c] = an[u][c];
         }
-        d.q[row] = acc;
+    }
+    double prod = 0.0;
+    if (own)
+    {
+        const size_t i = size_t(node) * 6 + a;
+        const v2f o = ds[i];
+        const float dn = d_next(beta, o.x, o.y);
+        pick2(d.dv, (k + 1) & 1)[i] = dn;
+        reinterpret_cast<float2 *>(pick2(d.mv, (k + 1) & 1))[i].x = dn;
+        d.q[i] = acc;
         prod = double(dn) * double(acc);
     }
-    const double tot = block_sum_192(prod, sh);
-    if (threadIdx.x == 0)
+    const double tot = wave_sum(prod);
+    if (lane == 0)
         part_dq[blockIdx.x] = tot;
 }
 
@@ -1100,7 +1154,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_dir(const SolveDesc *__rest
                                                          const double *__restrict__ part_rs)
 {
     __shared__ double sh[4];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const double delta = reduce_partials(part_rs, wg_begin[si], wg_begin[si + 1], sh);
     double beta = 0.0;
@@ -1122,7 +1176,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_dot(const SolveDesc *__rest
                                                          double *__restrict__ part_dq)
 {
     __shared__ double sh[4];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t node = (blockIdx.x - wg_begin[si]) * kPcgNodes + threadIdx.x / 6;
     double prod = 0.0;
@@ -1140,14 +1194,14 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_dot(const SolveDesc *__rest
 // (blockPCGSecondUpdateKernel, BlockPCG.cuh:125-169)
 __global__ __launch_bounds__(kPcgThreads) void k_pcg_update(const SolveDesc *__restrict__ sds,
                                                             const uint32_t *__restrict__ wg_begin, int n_solve, int k,
-                                                            const double *__restrict__ part_dq,
+                                                            uint32_t per, const double *__restrict__ part_dq,
                                                             double *__restrict__ part_rs)
 {
     __shared__ double sh[4];
     __shared__ float rb[kPcgThreads];
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
-    const double dq = reduce_partials(part_dq, wg_begin[si], wg_begin[si + 1], sh);
+    const double dq = reduce_partials(part_dq, wg_begin[si] * per, wg_begin[si + 1] * per, sh);
     const double alpha = (dq != 0.0) ? d.delta[k] / dq : 0.0;
     const float *__restrict__ dnew = pick2(d.dv, (k + 1) & 1);
     const uint32_t node = (blockIdx.x - wg_begin[si]) * kPcgNodes + threadIdx.x / 6;
@@ -1175,6 +1229,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_update(const SolveDesc *__r
             s += Mi[c] * double(rb[b0 + c]);
         const float sf = float(s);
         d.s[row] = sf;
+        reinterpret_cast<float2 *>(pick2(d.mv, (k + 1) & 1))[row].y = sf;
         prod = double(rn) * double(sf);
     }
     const double tot = block_sum_192(prod, sh);
@@ -1194,7 +1249,7 @@ __global__ void k_cost_final(const SolveDesc *__restrict__ sds, int slot)
 __global__ __launch_bounds__(256) void k_update(const SolveDesc *__restrict__ sds, const uint32_t *__restrict__ wg_begin,
                                                 int n_solve, int parity)
 {
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     if (blockIdx.x == wg_begin[si] && threadIdx.x < 64)
         reduce_cost(d, d.gn_iter + parity); // cost of the state this iteration started from
@@ -1206,7 +1261,7 @@ __global__ __launch_bounds__(256) void k_update(const SolveDesc *__restrict__ sd
 
 __global__ void k_identity(const SolveDesc *__restrict__ sds, const uint32_t *__restrict__ wg_begin, int n_solve)
 {
-    const int si = find_solve(wg_begin, n_solve, blockIdx.x);
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t n = (blockIdx.x - wg_begin[si]) * blockDim.x + threadIdx.x;
     if (n >= uint32_t(d.N))
@@ -1496,14 +1551,14 @@ hipError_t launch_pcg_init(const SolveDesc *sds, const uint32_t *wmap, int n_sol
 hipError_t launch_pcg_spmv(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
                            const double *part_rs, double *part_dq, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_pcg_spmv, dim3(n_wg), dim3(kPcgThreads), 0, st, sds, wmap, n_solve, k, part_rs, part_dq);
+    hipLaunchKernelGGL(k_pcg_spmv, dim3(n_wg * kPcgSpmvPer), dim3(64), 0, st, sds, wmap, n_solve, k, part_rs, part_dq);
     return hipGetLastError();
 }
 
 hipError_t launch_pcg_update(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
-                             const double *part_dq, double *part_rs, hipStream_t st)
+                             uint32_t per, const double *part_dq, double *part_rs, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_pcg_update, dim3(n_wg), dim3(kPcgThreads), 0, st, sds, wmap, n_solve, k, part_dq, part_rs);
+    hipLaunchKernelGGL(k_pcg_update, dim3(n_wg), dim3(kPcgThreads), 0, st, sds, wmap, n_solve, k, per, part_dq, part_rs);
     return hipGetLastError();
 }
 

@@ -120,8 +120,10 @@ hipError_t launch_pcg_init(const SolveDesc *sds, const uint32_t *wmap, int n_sol
                            hipStream_t st);
 hipError_t launch_pcg_spmv(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
                            const double *part_rs, double *part_dq, hipStream_t st);
+// per: partials of part_dq for each work-group of the map (kPcgSpmvPer after
+// launch_pcg_spmv, 1 after launch_pcg_dot)
 hipError_t launch_pcg_update(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
-                             const double *part_dq, double *part_rs, hipStream_t st);
+                             uint32_t per, const double *part_dq, double *part_rs, hipStream_t st);
 hipError_t launch_pcg_dir(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
                           const double *part_rs, hipStream_t st);
 hipError_t launch_pcg_dot(const SolveDesc *sds, const uint32_t *wmap, int n_solve, uint32_t n_wg, int k,
@@ -209,6 +211,7 @@ constexpr int kPartStride = 32;
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kWavesPerWg = 4;
 constexpr uint32_t kPcgNodesPerWg = 32;  // split PCG kernels
+constexpr uint32_t kPcgSpmvPer = 4;      // SpMV work-groups (and partials) for each of theirs: eight nodes
 
 // Forward warp of surfels and nodes (sh_warp.hip)
 // optical-flow input and node-motion prior (sh_flow.hip)
