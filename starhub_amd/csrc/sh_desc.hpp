@@ -74,6 +74,10 @@ struct SolveDesc
     int tile_pix;            // pixels per tile (64, 128 or 256) of the index build
     uint32_t *tile_cbase;    // n_tiles+1: first contribution of each tile
     uint32_t *tile_sbase;    // n_tiles+1: first slot of each tile
+    uint32_t *tile_nodes;    // n_tiles: distinct nodes of each tile (above kMatrixNodes: its slots are summed from lists)
+    uint8_t *gprank;         // P*K: each pixel slot's node as its rank in the tile (kNoRank: a later slot names it too)
+    uint16_t *tile_group;    // n_tiles*(kTileGroups+1): first slot of each 64-pixel group of a tile, then their end
+    uint16_t *slot_pair;     // S: the ranks of a slot's nodes, ra | rb << 8
     uint16_t *tc_contrib;    // contributions, per slot in pixel order: pixel | ka << 7 | kb << 10
     uint32_t *tc_slot_first; // S+1: first contribution of each slot
     uint32_t *list_off;      // N+2U+1: first entry of each block in list_items
@@ -166,6 +170,7 @@ __device__ __forceinline__ SolveDesc global_desc(const SolveDesc &src)
     SH_G(n2t_off); SH_G(n2t_terms);
     SH_G(half_keys); SH_G(half_off); SH_G(pair_entries); SH_G(upper_pos); SH_G(lower_pos); SH_G(row_ptr);
     SH_G(blk_col); SH_G(dense_cnt); SH_G(seg_ptr); SH_G(part); SH_G(tile_cbase); SH_G(tile_sbase);
+    SH_G(tile_nodes); SH_G(gprank); SH_G(tile_group); SH_G(slot_pair);
     SH_G(tc_contrib); SH_G(tc_slot_first); SH_G(list_off); SH_G(list_items); SH_G(slot_pos); SH_G(blk_transpose); SH_G(tpart);
     SH_G(dq[0]); SH_G(dq[1]); SH_G(jr); SH_G(reg); SH_G(ttrans); SH_G(blk); SH_G(dinv); SH_G(rhs);
     SH_G(x); SH_G(r); SH_G(s); SH_G(q); SH_G(dv[0]); SH_G(dv[1]); SH_G(mv[0]); SH_G(mv[1]);

@@ -181,6 +181,9 @@ int Engine::init(const sh_solver_config &c, uint32_t max_slots)
         A(d.seg_ptr, size_t(ncap_ + 1) * 4);
         A(d.tile_cbase, size_t(div_up(pcap_, kTilePixMin) + 1) * 4);
         A(d.tile_sbase, size_t(div_up(pcap_, kTilePixMin) + 1) * 4);
+        A(d.tile_nodes, size_t(div_up(pcap_, kTilePixMin)) * 4);
+        A(d.tile_group, size_t(div_up(pcap_, kTilePixMin)) * (kTileGroups + 1) * 2);
+        A(d.gprank, size_t(pcap_) * K_);
         A(d.list_off, (size_t(ncap_) + 2 * size_t(ucap_) + 1) * 4);
         A(d.blk_transpose, (size_t(ncap_) + 2 * size_t(ucap_)) * 4);
         A(d.jr, size_t(pcap_) * kHG * (fp16_ ? 2 : 4));
@@ -722,6 +725,7 @@ int Engine::build_group(const uint32_t *list, uint32_t n, hipStream_t st, int *r
                 if (r == SH_OK)
                 {
                     sl.tile_slot_max = d.n_tiles > 0 ? o[5] : 0u;
+                    sl.tiles_listed = d.n_tiles > 0 ? o[6] : 0u;
                     r = size_tiles(sl, o[3], o[4]);
                 }
                 n_slots[i] = o[3];
@@ -884,7 +888,8 @@ int Engine::size_tiles(Slot &sl, uint32_t n_slots, uint32_t n_contrib)
     const size_t b_first = up((size_t(n_slots) + 1) * 4);
     const size_t b_items = up(size_t(n_slots) * 4 + 4);
     const size_t b_part = up(size_t(n_slots) * kPartStride * 4 + 16); // 128-byte partials, 256-aligned base
-    const size_t need = b_contrib + b_first + 2 * b_items + b_part;
+    const size_t b_pair = up(size_t(n_slots) * 2 + 2);
+    const size_t need = b_contrib + b_first + 2 * b_items + b_part + b_pair;
     if (need > sl.tile_bytes)
         if (int rc = grow_buffer(&sl.tile_buf, &sl.tile_bytes, need + need / 4); rc != SH_OK)
             return rc;
@@ -894,6 +899,7 @@ int Engine::size_tiles(Slot &sl, uint32_t n_slots, uint32_t n_contrib)
     d.list_items = reinterpret_cast<uint32_t *>(b + b_contrib + b_first);
     d.tpart = reinterpret_cast<float *>(b + b_contrib + b_first + b_items);
     d.slot_pos = reinterpret_cast<uint32_t *>(b + b_contrib + b_first + b_items + b_part);
+    d.slot_pair = reinterpret_cast<uint16_t *>(b + b_contrib + b_first + 2 * b_items + b_part);
     return SH_OK;
 }
 
@@ -1011,7 +1017,7 @@ int Engine::enqueue_gn(uint32_t ns, hipStream_t st, uint32_t iters, bool identit
     const bool fp16 = fp16_;
     if (identity)
         SH_HIP(launch_identity(sds, map(kMapNode, ns), n, map_total_[kMapNode], st));
-    uint32_t max_n = 0, max_l = 0, tile = 1, slot_cap = 1;
+    uint32_t max_n = 0, max_l = 0, tile = 1, slot_cap = 1, n_listed = 0;
     const uint32_t *coop_begin = maps_.data() + size_t(kMapCoop) * (ns + 1);
     for (uint32_t s = 0; s < ns; ++s)
     {
@@ -1019,6 +1025,7 @@ int Engine::enqueue_gn(uint32_t ns, hipStream_t st, uint32_t iters, bool identit
         max_n = std::max(max_n, uint32_t(d.N));
         max_l = std::max(max_l, slots_[batch_[s]].max_row_len);
         slot_cap = std::max(slot_cap, slots_[batch_[s]].tile_slot_max);
+        n_listed += slots_[batch_[s]].tiles_listed;
         // blocks of one persistent-PCG group: its share plus one whole row
         const uint32_t G = coop_begin[s + 1] - coop_begin[s];
         const uint32_t nb = uint32_t(d.N) + 2u * uint32_t(d.U);
@@ -1101,7 +1108,7 @@ int Engine::enqueue_gn(uint32_t ns, hipStream_t st, uint32_t iters, bool identit
         {
             SH_HIP(mark(kPhTiles, st));
             SH_HIP(launch_tiles(K_, fp16, tile_pix(), fused, parity, sds, map(kMapTile, ns), n, map_total_[kMapTile],
-                                slot_cap, st));
+                                slot_cap, n_listed, st));
             SH_HIP(mark(kPhTilesCombine, st));
             SH_HIP(launch_tiles_combine(sds, map(kMapRow, ns), n, map_total_[kMapRow], tiles_lds, comb_wave,
                                         static_cast<PcgSlot2 *>(d_slots2_), pipe_slots, st));

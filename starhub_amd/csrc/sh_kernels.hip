@@ -358,6 +358,7 @@ __global__ void k_index_counts(IndexGroup g, int stage, IndexWs ws, uint32_t *ho
         o[3] = d.tile_sbase[nt];
         o[4] = d.tile_cbase[nt];
         o[5] = ws.tnslot[item.tc0 + nt + 1];
+        o[6] = ws.meta[size_t(it) * 16 + kMetaListed];
     }
 }
 

@@ -41,12 +41,13 @@ struct IndexGroup
 };
 // The group's workspace.  errs and the per-item meta words are cleared by the
 // kernels that read them last, so they are zero when the next build starts.
+constexpr uint32_t kMetaListed = 12;
 struct IndexWs
 {
     uint32_t *flags, *pos;         // raster valid flags and their exclusive scan
     uint32_t *tflags, *tpos;       // the same in tile order
     uint32_t *errs;                // one range-check word per item
-    uint32_t *meta;                // 16 words per item: [0] longest row
+    uint32_t *meta;                // 16 words per item: [0] longest row, [kMetaListed] tiles above kMatrixNodes
     uint32_t *bitmap;              // kBitmapWords per node key
     uint2 *bitpre;                 // the same words with the neighbour count of the words before each
     uint32_t *rowlen, *segcnt;     // per node key
@@ -86,7 +87,8 @@ hipError_t launch_n2t_split(const IndexGroup &g, const uint32_t *wmap, uint32_t 
 hipError_t launch_scan_jobs(const ScanJob *jobs, uint32_t n_jobs, hipStream_t st);
 // Counts for the host, host[item * 8 + k]: stage 1 -> [0] valid pixels,
 // [1] range-check flag (then cleared); stage 2 -> [0] segments, [1] longest
-// row, [2] U, [3] slots, [4] contributions, [5] largest tile slot count.
+// row, [2] U, [3] slots, [4] contributions, [5] largest tile slot count,
+// [6] tiles with more than kMatrixNodes nodes.
 hipError_t launch_index_counts(const IndexGroup &g, int stage, const IndexWs &ws, uint32_t *host, hipStream_t st);
 hipError_t launch_pair_kv(const SolveDesc &d, uint32_t *keys, uint32_t *vals, hipStream_t st);
 hipError_t launch_pair_heads(const uint32_t *keys, uint32_t n, uint32_t *head, uint32_t *meta, hipStream_t st);
@@ -249,6 +251,9 @@ hipError_t launch_forward_warp(uint32_t K, const float4 *warp, const float4 *ref
 
 // Pixel tiles (sh_tiles.hip): 64, 128 (default) or 256 pixels, per the tuning
 constexpr uint32_t kTilePixMin = 64, kTilePixDefault = 128, kTilePixMax = 256;
+constexpr uint32_t kTileGroups = kTilePixMax / 64; // 64-pixel groups of the largest tile
+// Distinct nodes of a tile whose slots the matrix form of the tile kernel sums.
+constexpr uint32_t kMatrixNodes = 64;
 // One work-group per tile: the tile's sorted contributions, slots and counts.
 hipError_t launch_tile_build(int K, uint32_t tile_pix, const IndexGroup &g, const uint32_t *wmap, uint32_t n_wg,
                              const IndexWs &ws, hipStream_t st);
@@ -263,8 +268,10 @@ hipError_t launch_block_transpose(const IndexGroup &g, const uint32_t *wmap, uin
 // fused: the tile kernel builds the FP32 per-pixel records itself (and the
 // dense cost partials) from the warp field of GN iteration offset parity,
 // instead of reading them; the term kernel then runs the ARAP part only.
+// n_listed: tiles of the launch with more than kMatrixNodes nodes.
 hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int parity, const SolveDesc *sds,
-                        const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, hipStream_t st);
+                        const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, uint32_t n_listed,
+                        hipStream_t st);
 // Longest row (blocks, diagonal included) the one-wave-per-row combine takes:
 // it holds a row's block sums in registers.
 constexpr uint32_t kWaveCombineMaxBlocks = 73;

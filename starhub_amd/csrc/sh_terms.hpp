@@ -53,6 +53,16 @@ __device__ __forceinline__ double dense_pixel_hg(const SolveDesc &d, uint32_t p,
     uint16_t kn[K];
     float w[K];
     load_knn<K>(d, p, kn, w);
+    const ushort4 px = d.gpix[p];
+    const uint32_t src = uint32_t(px.y) * uint32_t(d.W) + px.x;
+    const float4 cv = d.ref_v[src];
+    const float4 cn = d.ref_n[src];
+    // the measured texels too, before the warped vertex is known: their
+    // address needs the pixel pair only
+    const bool inside = px.z < d.W && px.w < d.H;
+    const uint32_t tgt = inside ? uint32_t(px.w) * uint32_t(d.W) + px.z : 0u;
+    const float4 tv4 = d.meas_v[tgt];
+    const float4 tn4 = d.meas_n[tgt];
     dq8 avg;
     avg.q0 = make_float4(0.f, 0.f, 0.f, 0.f);
     avg.q1 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -70,10 +80,6 @@ __device__ __forceinline__ double dense_pixel_hg(const SolveDesc &d, uint32_t p,
         avg.q1.w += w[k] * n.q1.w;
     }
     const rt34 T = dq_se3(avg);
-    const ushort4 px = d.gpix[p];
-    const uint32_t src = uint32_t(px.y) * uint32_t(d.W) + px.x;
-    const float4 cv = d.ref_v[src];
-    const float4 cn = d.ref_n[src];
     const f3 vw = rot_apply(T.r, mk3(cv.x, cv.y, cv.z)) + T.t;
     const f3 nw = rot_apply(T.r, mk3(cn.x, cn.y, cn.z));
     const f3 vc = rot_apply(d.w2c_r, vw) + mk3(d.w2c_t[0], d.w2c_t[1], d.w2c_t[2]);
@@ -82,11 +88,8 @@ __device__ __forceinline__ double dense_pixel_hg(const SolveDesc &d, uint32_t p,
 #pragma unroll
     for (int a = 0; a < 24; ++a)
         out[a] = 0.f;
-    if (px.z < d.W && px.w < d.H)
+    if (inside)
     {
-        const uint32_t tgt = uint32_t(px.w) * uint32_t(d.W) + px.z;
-        const float4 tv4 = d.meas_v[tgt];
-        const float4 tn4 = d.meas_n[tgt];
         const f3 tv = mk3(tv4.x, tv4.y, tv4.z), tn = mk3(tn4.x, tn4.y, tn4.z);
         bool ok = true;
         if (fabsf(tv4.x) < 1e-3f && fabsf(tv4.y) < 1e-3f && fabsf(tv4.z) < 1e-3f) // is_zero_vertex

@@ -163,6 +163,8 @@ __device__ __forceinline__ void group_min_max(uint32_t &lo, uint32_t &hi, uint32
     __syncthreads();
 }
 
+constexpr uint32_t kNoRank = 255u; // gprank: the slot adds nothing (a later slot of the pixel names its node)
+
 // ------------------------------------------------------------ index build
 // LDS of the tile build's ranking path: the tile's nodes and their ranks,
 // its node pairs (keys la * Dn + lb of the ranks la <= lb, Dn distinct nodes)
@@ -174,6 +176,7 @@ struct TileRankLds
     static constexpr int kPairWords = kMaxNodes * kMaxNodes / 32;
     static constexpr int kMaxPairs = 1024;  // distinct pairs of a tile on this path
     static constexpr int kMaskWords = TP / 32;
+    static constexpr int kGroups = (TP + kSlotPix - 1) / kSlotPix;
     static constexpr int kGroupWords = (kSlotPix < TP ? kSlotPix : TP) / 32; // mask words of a slot's pixel group
     uint32_t nbits[kBitmapWords];
     uint16_t npre[kBitmapWords];
@@ -182,7 +185,7 @@ struct TileRankLds
     uint16_t ppre[kPairWords];
     uint16_t pkey[kMaxPairs];
     uint32_t mask[kMaxPairs][kMaskWords];
-    uint16_t coff[kMaxPairs], soff[kMaxPairs];
+    uint16_t coff[kGroups][kMaxPairs]; // first contribution of each pair in each slot group
     uint32_t total[2];
 };
 
@@ -230,6 +233,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
         {
             tile_nslot[t] = 0;
             tile_ncontrib[t] = 0;
+            d.tile_nodes[t] = 0u;
         }
         return; // uniform over the group
     }
@@ -336,6 +340,20 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
         auto nrank = [&](uint32_t n) {
             return uint32_t(r.npre[n >> 5]) + uint32_t(__popc(r.nbits[n >> 5] & ((1u << (n & 31u)) - 1u)));
         };
+        // the pixel's nodes as ranks, half of them per thread (K = 8)
+        if constexpr (K == 8)
+            if (p < uint32_t(d.P))
+            {
+                uint32_t ranks = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    const bool on = half ? act[j + 4] : act[j];
+                    const uint32_t n = half ? kn[j + 4] : kn[j];
+                    ranks |= (on ? nrank(n) : kNoRank) << (8 * j);
+                }
+                reinterpret_cast<uint32_t *>(d.gprank)[size_t(p) * 2 + half] = ranks;
+            }
 #pragma unroll
         for (int i = 0; i < G::kItems; ++i)
             if (lohi[i] != 0xffffffffu)
@@ -374,67 +392,67 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
                     atomicOr(&r.mask[pk[i]][pl >> 5], 1u << (pl & 31u));
                 }
             __syncthreads();
-            // each pair's contribution count and slot count (non-empty
-            // kSlotPix-pixel groups), a run of pairs per thread, and their
-            // exclusive scans
+            // the slots (a pair's pixels of one kSlotPix-pixel group), group by
+            // group and by pair in each: contribution and slot counts of a
+            // run of pairs per thread, both in one word, and their exclusive
+            // scans (a group holds at most kSlotPix * kPairs contributions
+            // and kMaxPairs slots)
             const uint32_t per2 = (np + G::kThreads - 1) / G::kThreads;
             const uint32_t qb = min(np, tid * per2), qe = min(np, qb + per2);
-            uint32_t nc = 0, ns = 0;
-            for (uint32_t q = qb; q < qe; ++q)
+            uint32_t c_run[R::kGroups], s_run[R::kGroups], total_c = 0, total_s = 0;
 #pragma unroll
-                for (int w = 0; w < R::kMaskWords; ++w)
+            for (int gr = 0; gr < R::kGroups; ++gr)
+            {
+                uint32_t cnt = 0;
+                for (uint32_t q = qb; q < qe; ++q)
                 {
-                    const uint32_t m = r.mask[q][w];
-                    nc += __popc(m);
-                    if (w % R::kGroupWords == 0)
-                    {
-                        uint32_t grp = 0;
+                    uint32_t c = 0;
 #pragma unroll
-                        for (int w2 = 0; w2 < R::kGroupWords; ++w2)
-                            grp |= r.mask[q][w + w2];
-                        ns += grp ? 1u : 0u;
-                    }
+                    for (int w = 0; w < R::kGroupWords; ++w)
+                        c += __popc(r.mask[q][gr * R::kGroupWords + w]);
+                    cnt += c + (c ? 1u << 16 : 0u);
                 }
-            uint32_t total_c = 0, total_s = 0;
-            uint32_t c_run = group_exclusive_scan<G::kThreads>(nc, red, &total_c);
-            uint32_t s_run = group_exclusive_scan<G::kThreads>(ns, red, &total_s);
+                uint32_t all = 0;
+                const uint32_t before = group_exclusive_scan<G::kThreads>(cnt, red, &all);
+                c_run[gr] = total_c + (before & 0xffffu);
+                s_run[gr] = total_s + (before >> 16);
+                total_c += all & 0xffffu;
+                total_s += all >> 16;
+            }
             for (uint32_t q = qb; q < qe; ++q)
             {
-                r.coff[q] = uint16_t(c_run);
-                r.soff[q] = uint16_t(s_run);
                 // the pair's slots: block and first contribution
                 const uint32_t key = r.pkey[q];
                 const uint32_t lo = r.node_of[key / dn], hi = r.node_of[key % dn];
                 const uint32_t blk = block_of_pair(d.row_ptr, bitpre, lo, hi);
-                uint32_t c = c_run;
 #pragma unroll
-                for (int w = 0; w < R::kMaskWords; w += R::kGroupWords)
+                for (int gr = 0; gr < R::kGroups; ++gr)
                 {
                     uint32_t cnt = 0;
 #pragma unroll
-                    for (int w2 = 0; w2 < R::kGroupWords; ++w2)
-                        cnt += __popc(r.mask[q][w + w2]);
+                    for (int w = 0; w < R::kGroupWords; ++w)
+                        cnt += __popc(r.mask[q][gr * R::kGroupWords + w]);
+                    r.coff[gr][q] = uint16_t(c_run[gr]);
                     if (cnt)
                     {
-                        ws.tslot_block[tbase + s_run] = blk;
-                        ws.tslot_first[tbase + s_run] = uint16_t(c);
-                        ++s_run;
-                        c += cnt;
+                        ws.tslot_block[tbase + s_run[gr]] = blk;
+                        ws.tslot_first[tbase + s_run[gr]] = uint16_t(c_run[gr]);
+                        ++s_run[gr];
+                        c_run[gr] += cnt;
                     }
                 }
-                c_run = c;
             }
             __syncthreads();
-            // each contribution at its pair's first place plus the pair's pixels before it
+            // each contribution at its pair's first place in its group plus the pair's pixels before it there
 #pragma unroll
             for (int i = 0; i < G::kItems; ++i)
                 if (lohi[i] != 0xffffffffu)
                 {
-                    const uint32_t q = pk[i], pw = pl >> 5;
-                    uint32_t at = r.coff[q] + uint32_t(__popc(r.mask[q][pw] & ((1u << (pl & 31u)) - 1u)));
+                    const uint32_t q = pk[i], pw = pl >> 5, gw = pw / R::kGroupWords;
+                    uint32_t at = r.coff[gw][q] + uint32_t(__popc(r.mask[q][pw] & ((1u << (pl & 31u)) - 1u)));
 #pragma unroll
                     for (int w = 0; w < R::kMaskWords; ++w)
-                        if (uint32_t(w) < pw)
+                        if (uint32_t(w) < pw && uint32_t(w) / R::kGroupWords == gw)
                             at += __popc(r.mask[q][w]);
                     cout[at] = uint16_t(pl | (uint32_t(vals[i]) << kPixBits));
                 }
@@ -442,6 +460,9 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
             {
                 tile_nslot[t] = total_s;
                 tile_ncontrib[t] = total_c;
+                d.tile_nodes[t] = dn;
+                if (dn > kMatrixNodes)
+                    atomicAdd(ws.meta + size_t(it) * 16 + kMetaListed, 1u);
                 atomicMax(tile_nslot + uint32_t(d.n_tiles) + 1, total_s); // largest slot count of the solve's tiles
             }
             return; // uniform
@@ -520,6 +541,8 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
     {
         tile_nslot[t] = total_heads;
         tile_ncontrib[t] = total_valid; // valid items lead after the sort
+        d.tile_nodes[t] = 0xffffffffu;  // no ranks
+        atomicAdd(ws.meta + size_t(it) * 16 + kMetaListed, 1u);
         atomicMax(tile_nslot + uint32_t(d.n_tiles) + 1, total_heads); // largest slot count of the solve's tiles
     }
 }
@@ -571,6 +594,27 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_compact(IndexGroup g, con
         d.tc_slot_first[s0 + s] = c0 + ws.tslot_first[tbase + s];
         sort_keys[item.sb0 + s0 + s] = item.blk0 + ws.tslot_block[tbase + s];
         sort_vals[item.sb0 + s0 + s] = s0 + s;
+    }
+    // the matrix form's view of the tile: each slot's nodes as ranks (its
+    // first contribution's), and each 64-pixel group's first slot
+    if (K == 8 && d.tile_nodes[t] <= kMatrixNodes)
+    {
+        uint16_t *__restrict__ tg = d.tile_group + size_t(t) * (kTileGroups + 1);
+        if (ns == 0 && tid <= kTileGroups)
+            tg[tid] = 0;
+        for (uint32_t s = tid; s < ns; s += kTileThreads)
+        {
+            const uint32_t c = src[ws.tslot_first[tbase + s]];
+            const uint8_t *__restrict__ rk = d.gprank + (size_t(t) * TP + c_pix(c)) * K;
+            d.slot_pair[s0 + s] = uint16_t(rk[c_ka(c)] | (uint32_t(rk[c_kb(c)]) << 8));
+            const uint32_t g1 = c_pix(c) >> 6;
+            const uint32_t first = s == 0 ? 0u : (c_pix(src[ws.tslot_first[tbase + s - 1]]) >> 6) + 1u;
+            for (uint32_t gr = first; gr <= g1; ++gr)
+                tg[gr] = uint16_t(s);
+            if (s + 1 == ns)
+                for (uint32_t gr = g1 + 1; gr <= kTileGroups; ++gr)
+                    tg[gr] = uint16_t(ns);
+        }
     }
     if (t + 1 == uint32_t(d.n_tiles) && tid == 0)
         d.tc_slot_first[d.tile_sbase[t + 1]] = d.tile_cbase[t + 1];
@@ -632,6 +676,8 @@ __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ 
     const uint32_t t = blockIdx.x - wg_begin[si];
     if (t >= uint32_t(d.n_tiles))
         return; // uniform over the group
+    if (K == 8 && d.tile_nodes[t] <= kMatrixNodes)
+        return; // k_tiles_matrix sums this tile
     const uint32_t tid = threadIdx.x;
     const uint32_t p0 = t * TP;
     const uint32_t np = min(uint32_t(TP), uint32_t(d.P) - p0);
@@ -847,6 +893,179 @@ __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ 
             sum_slots(k, std::integral_constant<int, kTileRec / 4>{});
         else
             sum_slots(k, std::integral_constant<int, kTileRec / 4 - 1>{});
+    }
+}
+
+// The same sums as matrix products, for tiles of K = 8 with at most
+// kMatrixNodes nodes: a 64-pixel group's slots are C (slots x 64 pixels)
+// times its records (64 pixels x 28), C[(i, j), p] = w_i(p) w_j(p) and 0 where
+// the pixel does not name both nodes.  About half of C is not zero (a group
+// names some 13 nodes in 75 pairs), so the full product takes 2.2 times the
+// multiplications of the lists, at twice the vector rate, and reads the
+// records once per sixteen slots from registers instead of 112 bytes of LDS
+// per contribution: the list form is bound by that read and its bank
+// conflicts.  No list is read, and no slots are ordered by length.
+// v_mfma_f32_16x16x4_f32 adds its four products one after another, each fused
+// and rounded as fmaf, so over pixels in order (and zeros in between) a slot
+// has the list form's sum, bit for bit.
+// For K = 4 a pixel has ten pairs, not 36, and the lists are the better form.
+// Twelve solves of 128 to 4096 nodes: 186 us a launch from the lists, 147 us
+// so; 640x480 24.5 and 19.8 us; 1280x720 with FP16 records 44 and 33 us.  What
+// bounds it now is the chain of loads in front of a tile's records (work map,
+// descriptor, node ids, warp field) and the partials it writes.
+//
+// Pixel q of a group lies at column (q % 4) * 16 + q / 4 of the LDS rows: lane
+// quarter k takes pixels 4 s + k of step s, four steps in one 16-byte read.
+// A tile of up to 32 nodes holds its weights whole; with more nodes it goes
+// through its groups one at a time.
+template <class JT, int TP, bool FUSED>
+__global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__restrict__ sds,
+                                                         const uint32_t *__restrict__ wg_begin, int n_solve, int parity)
+{
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    constexpr int K = 8;
+    constexpr uint32_t NT = 2 * TP, kGroups = TP / 64;
+    constexpr uint32_t kHStride = TP + 4;                                       // floats between rows of Ht
+    constexpr uint32_t kW = 32 * (TP + 4) > 64 * 68 ? 32 * (TP + 4) : 64 * 68; // floats of the weight rows
+    static_assert(kMatrixNodes * 68 <= kW, "one group's weights of the largest tile");
+    __shared__ __align__(16) float Ht[kTileRec * kHStride]; // the records, a row per entry
+    __shared__ __align__(16) float Ws[kW];                  // the weights, a row per node
+    const int si = find_item(wg_begin, n_solve, blockIdx.x);
+    const SolveDesc d = global_desc(sds[si]);
+    const uint32_t t = blockIdx.x - wg_begin[si];
+    if (t >= uint32_t(d.n_tiles))
+        return; // uniform over the group
+    const uint32_t dn = d.tile_nodes[t];
+    if (dn > kMatrixNodes)
+        return; // k_tiles sums this tile from its lists
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t p0 = t * TP, np = min(uint32_t(TP), uint32_t(d.P) - p0);
+    const uint32_t s0 = d.tile_sbase[t];
+    const uint32_t c = lane & 15u, kq = lane >> 4, wave = tid >> 6; // operand row or column, step quarter
+    const bool whole = dn <= 32u; // every group's weights at once
+    const uint32_t per = whole ? kGroups : 1u, wstride = per * 64u + 4u;
+    // a group's slots, sixteen at a time, over its waves (two a group when
+    // whole, else all in turn): sixteen slots' nodes and partial places, read
+    // ahead of the sums (the first ones ahead of the records)
+    const uint32_t first = whole ? (wave & 1u) : wave, step = whole ? 2u : NT / 64u;
+    uint32_t pair, dst[4], m, se;
+    auto slots_at = [&](uint32_t at) __attribute__((always_inline)) {
+        pair = d.slot_pair[s0 + min(at + c, se - 1u)];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            dst[i] = d.slot_pos[s0 + min(at + 4u * kq + i, se - 1u)];
+    };
+    auto group_at = [&](uint32_t g) __attribute__((always_inline)) {
+        const uint16_t *__restrict__ tg = d.tile_group + size_t(t) * (kTileGroups + 1) + g;
+        m = tg[0] + 16u * first;
+        se = tg[1];
+        if (m < se)
+            slots_at(m);
+    };
+    group_at(whole ? wave >> 1 : 0u);
+    auto clear_weights = [&]() __attribute__((always_inline)) {
+        for (uint32_t i = tid; i < dn * wstride / 4u; i += NT)
+            reinterpret_cast<v4f *>(Ws)[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+    clear_weights();
+    float w[K];
+    uint32_t rank[2] = {0xffffffffu, 0xffffffffu};
+    double cost = 0.0;
+    const uint32_t q = tid & 63u, grp = tid >> 6, col = (q & 3u) * 16u + (q >> 2); // of the thread's pixel
+    if (tid < np)
+    {
+        const uint32_t p = p0 + tid;
+        const float4 *__restrict__ w4 = reinterpret_cast<const float4 *>(d.gpw + size_t(p) * K);
+        const float4 wa = w4[0], wb = w4[1];
+        const uint2 rk = reinterpret_cast<const uint2 *>(d.gprank)[p];
+        float hg[kHG];
+        if constexpr (FUSED)
+            cost = dense_pixel_hg<K>(d, p, parity, hg); // the record, built here instead of read
+        else
+            load_hg<JT>(d.jr, p, hg);
+#pragma unroll
+        for (int e = 0; e < kTileRec; ++e)
+            Ht[uint32_t(e) * kHStride + grp * 64u + col] = hg[e];
+        w[0] = wa.x, w[1] = wa.y, w[2] = wa.z, w[3] = wa.w;
+        w[4] = wb.x, w[5] = wb.y, w[6] = wb.z, w[7] = wb.w;
+        rank[0] = rk.x;
+        rank[1] = rk.y;
+    }
+    else if (tid < uint32_t(TP))
+#pragma unroll
+        for (int e = 0; e < kTileRec; ++e)
+            Ht[uint32_t(e) * kHStride + grp * 64u + col] = 0.f;
+    if constexpr (FUSED)
+    {
+        // the cost partials of the tile's 64-pixel groups, as the term kernel writes them
+        if (tid < uint32_t(TP))
+        {
+            const double wc = wave_sum(cost);
+            if (lane == 0 && p0 + tid < uint32_t(d.P))
+                d.cost_part[(p0 + tid) / 64u] = wc;
+        }
+    }
+    float *__restrict__ out = d.tpart;
+    for (uint32_t g0 = 0; g0 < kGroups; g0 += per)
+    {
+        if (g0)
+        {
+            __syncthreads(); // the group before is done with its weights
+            clear_weights();
+        }
+        __syncthreads();
+        if (tid < np && grp >= g0 && grp < g0 + per)
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+            {
+                const uint32_t r = (rank[k >> 2] >> (8 * (k & 3))) & 255u;
+                if (r != kNoRank)
+                    Ws[r * wstride + (grp - g0) * 64u + col] = w[k];
+            }
+        __syncthreads();
+        const uint32_t g = whole ? wave >> 1 : g0;
+        if (g0)
+            group_at(g);
+        if (m < se)
+        {
+            v4f h0[4], h1[4]; // records: entries c and 16 + c
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+            {
+                h0[j] = *reinterpret_cast<const v4f *>(Ht + c * kHStride + g * 64u + kq * 16u + 4u * j);
+                h1[j] = c < 12u ? *reinterpret_cast<const v4f *>(Ht + (16u + c) * kHStride + g * 64u + kq * 16u + 4u * j)
+                                : v4f{0.f, 0.f, 0.f, 0.f};
+            }
+            for (; m < se; m += 16u * step)
+            {
+                const float *__restrict__ wa = Ws + (pair & 255u) * wstride + (g - g0) * 64u + kq * 16u;
+                const float *__restrict__ wb = Ws + (pair >> 8) * wstride + (g - g0) * 64u + kq * 16u;
+                v4f a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+                const uint32_t to[4] = {dst[0], dst[1], dst[2], dst[3]};
+                if (m + 16u * step < se)
+                    slots_at(m + 16u * step);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                {
+                    const v4f x = reinterpret_cast<const v4f *>(wa)[j], y = reinterpret_cast<const v4f *>(wb)[j];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                    {
+                        const float coef = x[e] * y[e];
+                        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(coef, h0[j][e], a0, 0, 0, 0);
+                        a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(coef, h1[j][e], a1, 0, 0, 0);
+                    }
+                }
+                // lane quarter kq holds rows 4 kq .. 4 kq + 3, column c: a slot's partial is one 128-byte line
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i)
+                    if (m + 4u * kq + i < se)
+                    {
+                        out[size_t(to[i]) * kPartStride + c] = a0[i];
+                        out[size_t(to[i]) * kPartStride + 16u + c] = a1[i];
+                    }
+            }
+        }
     }
 }
 
@@ -1927,7 +2146,8 @@ hipError_t launch_block_transpose(const IndexGroup &g, const uint32_t *wmap, uin
 }
 
 hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int parity, const SolveDesc *sds,
-                        const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, hipStream_t st)
+                        const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, uint32_t n_listed,
+                        hipStream_t st)
 {
     if (n_wg == 0)
         return hipSuccess;
@@ -1938,15 +2158,28 @@ hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int par
     return with_tile_pix(tile_pix, [&](auto tp) {
         constexpr int TP = decltype(tp)::value;
         const dim3 grid(n_wg), block(2 * TP);
-        if (K == 8 && fused)
-            hipLaunchKernelGGL((k_tiles<8, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
-        else if (K == 8 && fp16)
-            hipLaunchKernelGGL((k_tiles<8, __half, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
-        else if (K == 8)
-            hipLaunchKernelGGL((k_tiles<8, float, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
+        if (K == 8)
+        {
+            if (fused)
+                hipLaunchKernelGGL((k_tiles_matrix<float, TP, true>), grid, block, 0, st, sds, wmap, n_solve, parity);
+            else if (fp16)
+                hipLaunchKernelGGL((k_tiles_matrix<__half, TP, false>), grid, block, 0, st, sds, wmap, n_solve,
+                                   parity);
+            else
+                hipLaunchKernelGGL((k_tiles_matrix<float, TP, false>), grid, block, 0, st, sds, wmap, n_solve,
+                                   parity);
+            if (n_listed == 0)
+                return;
+            if (fused)
+                hipLaunchKernelGGL((k_tiles<8, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
+                                   parity);
+            else if (fp16)
+                hipLaunchKernelGGL((k_tiles<8, __half, TP, false>), grid, block, lds, st, sds, wmap, n_solve,
+                                   slot_cap, parity);
+            else
+                hipLaunchKernelGGL((k_tiles<8, float, TP, false>), grid, block, lds, st, sds, wmap, n_solve,
+                                   slot_cap, parity);
+        }
         else if (fused)
             hipLaunchKernelGGL((k_tiles<4, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
                                parity);

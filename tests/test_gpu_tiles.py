@@ -1,0 +1,52 @@
+"""The tile kernel's matrix form against the row-segment path (no tiles), by the number of distinct nodes a tile
+names: up to 32 (a tile's weights whole), 33 to 64 (a group at a time), more (the list form, in the same launch), for
+every tile size, FP32 and FP16 records, and a last tile of a few pixels."""
+from dataclasses import replace
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("tile_pix", [64, 128, 256])
+def test_tiles_by_node_count(tile_pix, fp16):
+    import torch
+    from starhub_amd import native, scene, workload
+    assert torch.cuda.is_available()
+    torch.cuda.set_device(0)
+    flag = {64: native.SH_FLAG_TILE_PIX_64, 128: 0, 256: native.SH_FLAG_TILE_PIX_256}[tile_pix]
+    base = scene.config_c2()
+    cfg = replace(base, num_surfels=60000, num_nodes=700, width=331, height=203, fx=290.0, fy=290.0,
+                  solver=replace(base.solver, gn_iterations=1, fp16=fp16))
+    sc = scene.generate(cfg)
+    _, prod = workload.device_frame(sc)
+    K, N, idx = cfg.K, cfg.num_nodes, sc.index_map
+    rng = np.random.default_rng(tile_pix)
+    # bands of 64 columns whose surfels name nodes of one window each
+    knn = prod["surfel_knn"].reshape(-1, K).copy()
+    cover = 64 * np.arange(cfg.width // 64 + 1)
+    for x0, size in zip(cover, (8, 30, 33, 48, 64, 100)):
+        band = np.unique(idx[:, x0:x0 + 64])
+        for s in band[band != 0xFFFFFFFF]:
+            # eight different nodes: of a node named twice the tiles take the
+            # last slot and the row segments each of them
+            knn[s] = x0 + rng.choice(size, K, replace=False)
+    prod = dict(prod, surfel_knn=knn.reshape(prod["surfel_knn"].shape))
+
+    def solve(flags):
+        s = native.WarpSolver(native.make_config(cfg.solver, cfg.width, cfg.height, N, K, flags=flags))
+        f, _ = workload.device_frame(sc, producers=prod)
+        s.process_frame(f)
+        out = {n: s.debug(n, torch.float32).cpu().numpy() for n in ("blk", "rhs")}
+        s.close()
+        return out
+
+    tiled, rows = solve(flag), solve(native.SH_FLAG_ROW_SEGMENTS)
+    for name in ("blk", "rhs"):
+        a, b = tiled[name], rows[name]
+        print(tile_pix, fp16, name, "max diff", np.abs(a - b).max(), "max", np.abs(b).max(), flush=True)
+        # the same products of the same records in FP32, in another order: 168
+        # roundings of 2^-24 of the largest entry, all one way, reach 1e-5
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
