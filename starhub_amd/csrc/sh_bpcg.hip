@@ -6,15 +6,25 @@
 // call sequence: SetSolverInput(inv_diag, spmv, b, x) and
 // Solve(iterations, zero_init).
 //
-// Per iteration: the operator's q = A d (a host callback that enqueues on the
-// solve's stream, or the built-in block-CSR product), then three kernels:
-//   k_bp_dot     partial sums of d.q, one per work-group (FP64)
+// With the built-in block-CSR product an iteration is two kernels:
+//   k_bp_spmv    delta = t.s of the last update; beta = delta / delta_old;
+//                d = s + beta d where a row gathers it; q = A d; partials of d.q
 //   k_bp_update  alpha = delta / (d.q); x += alpha d; t = r - alpha q;
 //                s = M^-1 t; partial sums of t.s
-//   k_bp_dir     delta' = t.s; beta = delta' / delta; d = s + beta d
+// With an operator of the caller's (a host callback that enqueues on the
+// solve's stream) the product needs d in memory, and it is four, to the same
+// bits: the callback, k_bp_dot (partials of d.q), k_bp_update, k_bp_dir (d).
+// Bound by launches and by the latency of each kernel's dependent loads, not
+// by bandwidth: one lane per scalar row of a block, so that loads are
+// contiguous over six lanes, five lanes to a scalar row's blocks in the
+// product, and all of a lane's loads in flight before partials are summed.
+// Of more than 8192 rows a work-group takes several turns, so that the update
+// has at most 1024 partials to sum.  With one thread per 6-row block and a row's blocks one after another
+// in four kernels, 256 rows and 10 iterations took 179 us and 4096 rows and 20
+// iterations 366 us; 114 and 220 us so.
 // Every work-group reduces the same partials in the same order, so alpha and
 // beta are the same bits everywhere; vectors are FP32 as in the reference,
-// dot products, alpha and beta FP64 (cuBLAS Sdot in the reference,
+// the product's row sums, dot products, alpha and beta FP64 (cuBLAS Sdot in the reference,
 // BlockPCG.cuh:418-471).  A zero system gives alpha = beta = 0 instead of 0/0.
 #include <algorithm>
 #include <cmath>
@@ -30,23 +40,75 @@ namespace sh
 {
 namespace
 {
-constexpr int kBpThreads = 256; // one 6-row block per thread
+constexpr int kBpThreads = 256;
+constexpr int kBpWaveRows = 10;                               // 6-row blocks of a wave: 60 lanes, one scalar row each
+constexpr int kBpGroupRows = kBpWaveRows * (kBpThreads / 64); // and of a work-group
+// The product: two rows a wave, five blocks of each at a time (a lane holds
+// one scalar row of a block), kBpAhead of these in flight.  20 iterations with
+// 16 blocks a row, 256 / 4096 / 20000 rows: 211 / 226 / 419 us with two in
+// flight, 207 / 233 / 462 with three, 212 / 237 / 504 with four (136
+// registers, fewer waves); one lane per scalar row of the system with its
+// blocks one after another 240 / 282 us at 256 and 4096 rows; work-groups of
+// 512 and 1024 threads are slower at 256 rows (121 and 141 for 101 us at 10
+// iterations).
+constexpr int kBpRowBlocks = 5;
+constexpr int kBpRowLanes = 6 * kBpRowBlocks;
+constexpr int kBpAhead = 2;
+constexpr int kBpSpmvThreads = 256;
+constexpr int kBpSpmvRows = 2 * (kBpSpmvThreads / 64); // rows of a work-group in one turn
+constexpr uint32_t kBpSpmvGroups = 1024;           // more rows than these take turns
+
+// A lane's scalar row: row 6 * row + a of the system, in the wave's lane 6 * (row of the wave) + a
+struct BpLane
+{
+    uint32_t row, a, i; // clamped to the last row where off
+    int first;          // the lane of the block's first row
+    bool on;
+};
+
+__device__ inline BpLane bp_lane(uint32_t nblk)
+{
+    const uint32_t lane = threadIdx.x % 64u, wave = threadIdx.x / 64u;
+    BpLane l;
+    l.a = lane % 6u;
+    l.first = int(lane - l.a);
+    const uint32_t row = blockIdx.x * kBpGroupRows + wave * kBpWaveRows + lane / 6u;
+    l.on = lane < 6u * kBpWaveRows && row < nblk;
+    l.row = min(row, nblk - 1u);
+    l.i = 6u * l.row + l.a;
+    return l;
+}
 
 // Sum of `n` FP64 partials in a fixed order (lane j takes j, j+64, ...; then a
-// fixed shuffle tree); every wave that calls it gets the same bits.
-__device__ inline double sum_partials(const double *__restrict__ part, uint32_t n)
+// fixed shuffle tree); every wave that calls it gets the same bits.  Eight
+// loads in flight, past the end the last partial again.
+__device__ inline double lane_partials(const double *__restrict__ part, uint32_t n)
 {
     double v = 0.0;
-    for (uint32_t i = threadIdx.x % 64u; i < n; i += 64)
-        v += part[i];
-    return wave_sum(v);
+    for (uint32_t i = threadIdx.x % 64u; i < n; i += 8 * 64)
+    {
+        double p[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            p[u] = part[min(i + 64u * u, n - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            v = i + 64u * u < n ? v + p[u] : v;
+    }
+    return v;
+}
+
+__device__ inline double sum_partials(const double *__restrict__ part, uint32_t n)
+{
+    return wave_sum(lane_partials(part, n));
 }
 
 // Work-group sum of one value per thread, in a fixed order: wave sums, then
 // the waves' sums in wave order.  Written by thread 0 to out.
+template <int THREADS = kBpThreads>
 __device__ inline void block_sum_store(double v, double *__restrict__ out)
 {
-    __shared__ double ws[kBpThreads / 64];
+    __shared__ double ws[THREADS / 64];
     v = wave_sum(v);
     if (threadIdx.x % 64u == 0)
         ws[threadIdx.x / 64u] = v;
@@ -54,71 +116,64 @@ __device__ inline void block_sum_store(double v, double *__restrict__ out)
     if (threadIdx.x == 0)
     {
         double s = 0.0;
-        for (int w = 0; w < kBpThreads / 64; ++w)
+        for (int w = 0; w < THREADS / 64; ++w)
             s += ws[w];
         *out = s;
     }
 }
 
-// y = M^-1 v for 6-row block b (M^-1: 36 FP32 per block, row-major), FP64 accumulation
-__device__ inline void precond6(const float *__restrict__ minv, const float *__restrict__ v, uint32_t b, float *y)
+// this lane's row of M^-1 (36 FP32 per block, row-major) and its product with
+// v, FP64 accumulation; v: the lane's own entry, the block's others from its lanes
+struct BpInvRow
 {
-    float vb[6];
+    float m[6];
+};
+
+__device__ inline BpInvRow load_inv(const float *__restrict__ minv, const BpLane &l)
+{
+    BpInvRow mi;
 #pragma unroll
     for (int j = 0; j < 6; ++j)
-        vb[j] = v[6 * size_t(b) + j];
-    const float *m = minv + 36 * size_t(b);
-#pragma unroll
-    for (int i = 0; i < 6; ++i)
-    {
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < 6; ++j)
-            acc += double(m[6 * i + j]) * double(vb[j]);
-        y[i] = float(acc);
-    }
+        mi.m[j] = minv[6 * size_t(l.i) + j];
+    return mi;
 }
 
-__device__ inline double dot6(const float *a, const float *__restrict__ v, uint32_t b)
+__device__ inline float precond6(const BpInvRow &mi, float v, const BpLane &l)
 {
     double acc = 0.0;
 #pragma unroll
     for (int j = 0; j < 6; ++j)
-        acc += double(a[j]) * double(v[6 * size_t(b) + j]);
-    return acc;
+        acc += double(mi.m[j]) * double(__shfl(v, l.first + j, 64));
+    return float(acc);
 }
 
-// r = b, x = 0 (zero_init) or r given (InitResidual already ran); d = M^-1 r;
-// partials of r.d  (blockPCGZeroInitKernel / Initialize, BlockPCG.cuh:395-440)
+// r = b, x = 0 (zero_init) or r given (InitResidual already ran); s = M^-1 r;
+// partials of r.s  (blockPCGZeroInitKernel / Initialize, BlockPCG.cuh:395-440)
 __global__ void k_bp_init(const float *__restrict__ b, const float *__restrict__ minv, float *__restrict__ r,
-                          float *__restrict__ d, float *__restrict__ x, uint32_t nblk, int zero_init,
+                          float *__restrict__ s, float *__restrict__ x, uint32_t nblk, int zero_init,
                           double *__restrict__ part)
 {
-    const uint32_t blk = blockIdx.x * kBpThreads + threadIdx.x;
-    double v = 0.0;
-    if (blk < nblk)
+    const BpLane l = bp_lane(nblk);
+    const float rv = zero_init ? b[l.i] : r[l.i];
+    const float y = precond6(load_inv(minv, l), rv, l);
+    if (l.on)
     {
         if (zero_init)
-            for (int j = 0; j < 6; ++j)
-            {
-                r[6 * size_t(blk) + j] = b[6 * size_t(blk) + j];
-                x[6 * size_t(blk) + j] = 0.f;
-            }
-        float y[6];
-        precond6(minv, r, blk, y);
-        for (int j = 0; j < 6; ++j)
-            d[6 * size_t(blk) + j] = y[j];
-        v = dot6(y, r, blk);
+        {
+            r[l.i] = rv;
+            x[l.i] = 0.f;
+        }
+        s[l.i] = y;
     }
-    block_sum_store(v, part + blockIdx.x);
+    block_sum_store(l.on ? double(y) * double(rv) : 0.0, part + blockIdx.x);
 }
 
-// delta[0] = sum of the init partials (one wave)
-__global__ void k_bp_delta0(const double *__restrict__ part, uint32_t n, double *__restrict__ delta)
+// delta[it] = sum of the partials (one wave)
+__global__ void k_bp_delta(const double *__restrict__ part, uint32_t n, double *__restrict__ delta, uint32_t it)
 {
     const double s = sum_partials(part, n);
     if (threadIdx.x == 0)
-        delta[0] = s;
+        delta[it] = s;
 }
 
 // r = b - y  (InitResidual through ApplySpMV when the operator has no InitResidual)
@@ -129,103 +184,240 @@ __global__ void k_bp_sub(const float *__restrict__ b, const float *__restrict__ 
         r[i] = b[i] - y[i];
 }
 
+// A lane's place in the product: row r of the wave's two, blocks j, j + 5, ...
+// of it, scalar row a; lead: a lane that holds a scalar row's sum
+struct BpRowLane
+{
+    uint32_t r, j, a;
+    bool lead;
+};
+
+__device__ inline BpRowLane bp_row_lane()
+{
+    const uint32_t lane = threadIdx.x % 64u;
+    BpRowLane l;
+    l.r = min(lane / uint32_t(kBpRowLanes), 1u); // the last four lanes repeat row 1 and sum nothing
+    const uint32_t e = lane - l.r * kBpRowLanes;
+    l.j = e / 6u;
+    l.a = e % 6u;
+    l.lead = l.j == 0u;
+    return l;
+}
+
+// the dot product d.q over the lanes and turns of k_bp_spmv
 __global__ void k_bp_dot(const float *__restrict__ d, const float *__restrict__ q, uint32_t nblk,
                          double *__restrict__ part)
 {
-    const uint32_t blk = blockIdx.x * kBpThreads + threadIdx.x;
+    const BpRowLane l = bp_row_lane();
     double v = 0.0;
-    if (blk < nblk)
+    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nblk; row0 += gridDim.x * kBpSpmvRows)
     {
-        float db[6];
-        for (int j = 0; j < 6; ++j)
-            db[j] = d[6 * size_t(blk) + j];
-        v = dot6(db, q, blk);
+        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+        if (l.lead && row < nblk)
+            v += double(d[6 * size_t(row) + l.a]) * double(q[6 * size_t(row) + l.a]);
     }
-    block_sum_store(v, part + blockIdx.x);
+    block_sum_store<kBpSpmvThreads>(v, part + blockIdx.x);
 }
 
 // the second kernel of the reference's iteration (BlockPCG.cuh:442-472)
 __global__ void k_bp_update(float *__restrict__ x, const float *__restrict__ r, const float *__restrict__ d,
                             const float *__restrict__ q, const float *__restrict__ minv, float *__restrict__ t,
                             float *__restrict__ s, uint32_t nblk, const double *__restrict__ part_dq,
-                            const double *__restrict__ delta, uint32_t it, double *__restrict__ part_ts)
+                            uint32_t n_dq, const double *__restrict__ delta, uint32_t it,
+                            double *__restrict__ part_ts)
 {
-    __shared__ double alpha_sh;
-    if (threadIdx.x < 64)
+    const BpLane l = bp_lane(nblk);
+    // everything is loaded before the partials are summed
+    const double delta_it = delta[it];
+    const float xv = x[l.i], rv = r[l.i], dv = d[l.i], qv = q[l.i];
+    const BpInvRow mi = load_inv(minv, l);
+    const double dq = sum_partials(part_dq, n_dq);
+    const float a = float(dq != 0.0 ? delta_it / dq : 0.0);
+    const float tv = rv - a * qv;
+    const float y = precond6(mi, tv, l);
+    if (l.on)
     {
-        const double dq = sum_partials(part_dq, gridDim.x);
-        if (threadIdx.x == 0)
-            alpha_sh = dq != 0.0 ? delta[it] / dq : 0.0;
+        x[l.i] = xv + a * dv;
+        t[l.i] = tv;
+        s[l.i] = y;
     }
-    __syncthreads();
-    const double alpha = alpha_sh;
-    const uint32_t blk = blockIdx.x * kBpThreads + threadIdx.x;
-    double v = 0.0;
-    if (blk < nblk)
-    {
-        const float a = float(alpha);
-        for (int j = 0; j < 6; ++j)
-        {
-            const size_t i = 6 * size_t(blk) + j;
-            x[i] = x[i] + a * d[i];
-            t[i] = r[i] - a * q[i];
-        }
-        float y[6];
-        precond6(minv, t, blk, y);
-        for (int j = 0; j < 6; ++j)
-            s[6 * size_t(blk) + j] = y[j];
-        v = dot6(y, t, blk);
-    }
-    block_sum_store(v, part_ts + blockIdx.x);
+    block_sum_store(l.on ? double(y) * double(tv) : 0.0, part_ts + blockIdx.x);
 }
 
-// the third kernel (BlockPCG.cuh:474-483): d = s + beta d; delta[it+1] = t.s
+// delta' = t.s and beta = delta' / delta of iteration it, by a whole wave from
+// its lanes' sums; the first work-group keeps delta' for the update and the history
+__device__ inline float bp_beta(double lane_sum, double *__restrict__ delta, uint32_t it)
+{
+    const double dold = it ? delta[it - 1] : 0.0;
+    const double dn = wave_sum(lane_sum);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        delta[it] = dn;
+    return float(dold != 0.0 ? dn / dold : 0.0);
+}
+
+// the third kernel (BlockPCG.cuh:474-483): d = s + beta d; delta[it] = t.s (iteration 0: d = s)
 __global__ void k_bp_dir(const float *__restrict__ s, float *__restrict__ d, uint32_t nblk,
                          const double *__restrict__ part_ts, double *__restrict__ delta, uint32_t it)
 {
-    __shared__ double beta_sh;
-    if (threadIdx.x < 64)
-    {
-        const double dn = sum_partials(part_ts, gridDim.x);
-        if (threadIdx.x == 0)
-        {
-            const double dold = delta[it];
-            beta_sh = dold != 0.0 ? dn / dold : 0.0;
-            if (blockIdx.x == 0)
-                delta[it + 1] = dn;
-        }
-    }
-    __syncthreads();
-    const float beta = float(beta_sh);
-    const uint32_t blk = blockIdx.x * kBpThreads + threadIdx.x;
-    if (blk < nblk)
-        for (int j = 0; j < 6; ++j)
-        {
-            const size_t i = 6 * size_t(blk) + j;
-            d[i] = s[i] + beta * d[i];
-        }
+    const BpLane l = bp_lane(nblk);
+    const float beta = bp_beta(lane_partials(part_ts, gridDim.x), delta, it);
+    if (l.on)
+        d[l.i] = it ? s[l.i] + beta * d[l.i] : s[l.i];
 }
 
-// y = A x over a 6x6 block-CSR (row-major blocks), one thread per scalar row,
-// blocks of a row in storage order (performSparseMVKernel, ApplySpMVBinBlockCSR.cuh:13-60)
-__global__ void k_bcsr_spmv(const uint32_t *__restrict__ row_ptr, const uint32_t *__restrict__ col,
-                            const float *__restrict__ blocks, const float *__restrict__ x, const float *__restrict__ b,
-                            float *__restrict__ y, uint32_t nrows)
+struct BpVector // a vector in memory
 {
-    const uint32_t i = blockIdx.x * kBpThreads + threadIdx.x;
-    if (i >= 6 * nrows)
-        return;
-    const uint32_t row = i / 6u, a = i % 6u;
-    float acc = 0.f;
-    for (uint32_t k = row_ptr[row]; k < row_ptr[row + 1]; ++k)
+    struct Entries
     {
-        const float *blk = blocks + 36 * size_t(k) + 6 * a;
-        const float *xv = x + 6 * size_t(col[k]);
+        float x[6];
+    };
+    const float *__restrict__ x;
+    __device__ void load(uint32_t col, Entries &e) const
+    {
 #pragma unroll
         for (int c = 0; c < 6; ++c)
-            acc += blk[c] * xv[c];
+            e.x[c] = x[6 * size_t(col) + c];
     }
-    y[i] = b ? b[i] - acc : acc; // b: InitResidual's r = b - A x
+    __device__ float value(const Entries &e, int c) const { return e.x[c]; }
+};
+
+struct BpDirection // d = s + beta d_old (iteration 0: s)
+{
+    struct Entries
+    {
+        float s[6], d[6];
+    };
+    const float *__restrict__ s, *__restrict__ d;
+    bool old;
+    float beta;
+    __device__ void load(uint32_t col, Entries &e) const
+    {
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+            e.s[c] = s[6 * size_t(col) + c];
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+            e.d[c] = d[6 * size_t(col) + c];
+    }
+    __device__ float value(const Entries &e, int c) const { return old ? e.s[c] + beta * e.d[c] : e.s[c]; }
+};
+
+// Scalar row 6 * row + a of A v over a 6x6 block-CSR (row-major blocks;
+// performSparseMVKernel, ApplySpMVBinBlockCSR.cuh:13-60), in FP64, rounded
+// once; valid in the row's lead lanes.  Five lanes share a scalar row, each
+// with kBpAhead blocks in flight, so that a row of up to ten blocks costs one
+// trip to memory after its columns; past the row's end the last block is
+// loaded again and not summed.  ready() runs in the whole wave when the first
+// blocks are in flight.
+template <class V, class F>
+__device__ inline float bcsr_row(const uint32_t *__restrict__ row_ptr, const uint32_t *__restrict__ col,
+                                 const float *__restrict__ blocks, uint32_t row, const BpRowLane &l, V &v, F ready)
+{
+    const uint32_t k0 = row_ptr[row], k1 = row_ptr[row + 1];
+    const uint32_t last = k1 > k0 ? k1 - 1u : 0u; // an empty row loads block 0 (there is one) and sums nothing
+    float m[kBpAhead][6];
+    typename V::Entries e[kBpAhead];
+    auto load = [&](uint32_t k) __attribute__((always_inline)) {
+        uint32_t cols[kBpAhead];
+#pragma unroll
+        for (int u = 0; u < kBpAhead; ++u)
+            cols[u] = col[min(k + u * kBpRowBlocks, last)];
+#pragma unroll
+        for (int u = 0; u < kBpAhead; ++u)
+        {
+            const float *blk = blocks + 36 * size_t(min(k + u * kBpRowBlocks, last)) + 6 * l.a;
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+                m[u][c] = blk[c];
+        }
+#pragma unroll
+        for (int u = 0; u < kBpAhead; ++u)
+            v.load(cols[u], e[u]);
+    };
+    double acc = 0.0;
+    auto sum = [&](uint32_t k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < kBpAhead; ++u)
+        {
+            double with = acc;
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+                with = fma(double(m[u][c]), double(v.value(e[u], c)), with);
+            acc = k + u * kBpRowBlocks < k1 ? with : acc;
+        }
+    };
+    uint32_t k = k0 + l.j;
+    load(k);
+    ready();
+    sum(k);
+#pragma unroll 1
+    for (k += kBpAhead * kBpRowBlocks; k < k1; k += kBpAhead * kBpRowBlocks)
+    {
+        load(k);
+        sum(k);
+    }
+    // the row's five sums, in the lanes of the first
+    const int lane = int(threadIdx.x % 64u);
+    const double pair = acc + __shfl(acc, lane + 12, 64);
+    const double fifth = __shfl(acc, lane + 24, 64);
+    return float(pair + __shfl(pair, lane + 6, 64) + fifth);
+}
+
+// y = A x, or y = b - A x (b: InitResidual's r = b - A x)
+__global__ __launch_bounds__(kBpSpmvThreads) void k_bcsr_spmv(const uint32_t *__restrict__ row_ptr,
+                                                          const uint32_t *__restrict__ col,
+                                                          const float *__restrict__ blocks, const float *__restrict__ x,
+                                                          const float *__restrict__ b, float *__restrict__ y,
+                                                          uint32_t nrows)
+{
+    const BpRowLane l = bp_row_lane();
+    const BpVector v{x};
+    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nrows; row0 += gridDim.x * kBpSpmvRows)
+    {
+        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+        const size_t i = 6 * size_t(row) + l.a;
+        const float acc = bcsr_row(row_ptr, col, blocks, min(row, nrows - 1u), l, v, [] {});
+        if (l.lead && row < nrows)
+            y[i] = b ? b[i] - acc : acc;
+    }
+}
+
+// k_bp_dir, k_bcsr_spmv and k_bp_dot in one: the direction is formed where it
+// is gathered, from s and the old direction, and each row stores its own part
+// of the new one (another buffer: other rows still read the old)
+__global__ __launch_bounds__(kBpSpmvThreads) void k_bp_spmv(const uint32_t *__restrict__ row_ptr,
+                                                        const uint32_t *__restrict__ col,
+                                                        const float *__restrict__ blocks, const float *__restrict__ s,
+                                                        const float *__restrict__ d_old, float *__restrict__ d,
+                                                        float *__restrict__ q, uint32_t nblk,
+                                                        const double *__restrict__ part_ts, uint32_t n_ts,
+                                                        double *__restrict__ delta, uint32_t it,
+                                                        double *__restrict__ part_dq)
+{
+    const BpRowLane l = bp_row_lane();
+    const double ts = lane_partials(part_ts, n_ts);
+    BpDirection v{s, it ? d_old : s, it != 0u, 0.f};
+    bool first = true;
+    double dq = 0.0;
+    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nblk; row0 += gridDim.x * kBpSpmvRows)
+    {
+        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+        const size_t i = 6 * size_t(min(row, nblk - 1u)) + l.a;
+        const float sv = s[i], ov = v.d[i];
+        const float acc = bcsr_row(row_ptr, col, blocks, min(row, nblk - 1u), l, v, [&] {
+            if (first)
+                v.beta = bp_beta(ts, delta, it);
+            first = false;
+        });
+        if (l.lead && row < nblk)
+        {
+            const float dv = it ? sv + v.beta * ov : sv;
+            d[i] = dv;
+            q[i] = acc;
+            dq += double(dv) * double(acc);
+        }
+    }
+    block_sum_store<kBpSpmvThreads>(dq, part_dq + blockIdx.x);
 }
 
 __global__ void k_bcsr_check(const uint32_t *__restrict__ row_ptr, const uint32_t *__restrict__ col, uint32_t nrows,
@@ -246,6 +438,11 @@ __global__ void k_bcsr_check(const uint32_t *__restrict__ row_ptr, const uint32_
 }
 
 inline uint32_t grid_of(uint32_t n) { return (n + kBpThreads - 1) / kBpThreads; }
+inline uint32_t spmv_grid(uint32_t nblk)
+{
+    return std::min((nblk + kBpSpmvRows - 1) / kBpSpmvRows, kBpSpmvGroups);
+}
+inline uint32_t row_grid(uint32_t nblk) { return (nblk + kBpGroupRows - 1) / kBpGroupRows; }
 
 int status_of(hipError_t e)
 {
@@ -267,7 +464,8 @@ struct sh_spmv
 struct sh_block_pcg
 {
     uint32_t cap = 0; // max_matrix_size
-    float *r = nullptr, *t = nullptr, *d = nullptr, *q = nullptr, *s = nullptr;
+    void *block = nullptr; // one allocation for the vectors and partials
+    float *r = nullptr, *t = nullptr, *d = nullptr, *d_old = nullptr, *q = nullptr, *s = nullptr;
     double *part_a = nullptr, *part_b = nullptr, *delta = nullptr;
     uint32_t max_iters = 0;  // delta holds max_iters + 1 entries
     uint32_t last_iters = 0; // iterations the last solve ran
@@ -283,11 +481,10 @@ namespace
 {
 void bpcg_free(sh_block_pcg *p)
 {
-    for (void *a : {static_cast<void *>(p->r), static_cast<void *>(p->t), static_cast<void *>(p->d),
-                    static_cast<void *>(p->q), static_cast<void *>(p->s), static_cast<void *>(p->part_a),
-                    static_cast<void *>(p->part_b), static_cast<void *>(p->delta)})
-        if (a)
-            (void)hipFree(a);
+    if (p->block)
+        (void)hipFree(p->block);
+    if (p->delta)
+        (void)hipFree(p->delta);
     delete p;
 }
 
@@ -363,7 +560,7 @@ extern "C"
     {
         if (!spmv || !x || !y)
             return SH_E_ARG;
-        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::grid_of(6u * spmv->rows)), dim3(sh::kBpThreads), 0,
+        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::spmv_grid(spmv->rows)), dim3(sh::kBpSpmvThreads), 0,
                            reinterpret_cast<hipStream_t>(stream), spmv->row_ptr, spmv->col, spmv->blocks, x,
                            static_cast<const float *>(nullptr), y, spmv->rows);
         return sh::status_of(hipGetLastError());
@@ -374,7 +571,7 @@ extern "C"
     {
         if (!spmv || !x_init || !b || !residual)
             return SH_E_ARG;
-        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::grid_of(6u * spmv->rows)), dim3(sh::kBpThreads), 0,
+        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::spmv_grid(spmv->rows)), dim3(sh::kBpSpmvThreads), 0,
                            reinterpret_cast<hipStream_t>(stream), spmv->row_ptr, spmv->col, spmv->blocks, x_init, b,
                            residual, spmv->rows);
         return sh::status_of(hipGetLastError());
@@ -407,12 +604,14 @@ extern "C"
             return SH_E_ARG;
         sh_block_pcg *p = new sh_block_pcg();
         p->cap = max_matrix_size;
-        const size_t vb = size_t(max_matrix_size) * 4;
-        const size_t pb = size_t(sh::grid_of(max_matrix_size / 6u)) * 8;
-        bool ok = hipMalloc(&p->r, vb) == hipSuccess && hipMalloc(&p->t, vb) == hipSuccess &&
-                  hipMalloc(&p->d, vb) == hipSuccess && hipMalloc(&p->q, vb) == hipSuccess &&
-                  hipMalloc(&p->s, vb) == hipSuccess && hipMalloc(&p->part_a, pb) == hipSuccess &&
-                  hipMalloc(&p->part_b, pb) == hipSuccess && ensure_delta(p, 16) == SH_OK;
+        const size_t vb = (size_t(max_matrix_size) * 4 + 255) / 256 * 256; // a vector's stride
+        const size_t na = sh::spmv_grid(max_matrix_size / 6u), nb = sh::row_grid(max_matrix_size / 6u);
+        const bool ok = hipMalloc(&p->block, 6 * vb + (na + nb) * 8) == hipSuccess && ensure_delta(p, 16) == SH_OK;
+        float **const vec[6] = {&p->r, &p->t, &p->d, &p->d_old, &p->q, &p->s};
+        for (int i = 0; ok && i < 6; ++i)
+            *vec[i] = reinterpret_cast<float *>(static_cast<char *>(p->block) + i * vb);
+        p->part_a = ok ? reinterpret_cast<double *>(static_cast<char *>(p->block) + 6 * vb) : nullptr;
+        p->part_b = ok ? p->part_a + na : nullptr;
         if (!ok)
         {
             bpcg_free(p);
@@ -462,7 +661,7 @@ extern "C"
         if (rc != SH_OK)
             return rc;
         const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-        const uint32_t nblk = pcg->n / 6u, g = sh::grid_of(nblk);
+        const uint32_t nblk = pcg->n / 6u, g = sh::row_grid(nblk), gq = sh::spmv_grid(nblk);
         pcg->last_iters = 0;
         if (!zero_init)
         {
@@ -478,29 +677,53 @@ extern "C"
             if (rc != SH_OK)
                 return rc;
         }
+        // s = M^-1 r and the partials of r.s; each iteration begins with their sum
         hipLaunchKernelGGL(sh::k_bp_init, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->b, pcg->inv_diag, pcg->r,
-                           pcg->d, pcg->x, nblk, zero_init ? 1 : 0, pcg->part_a);
-        hipLaunchKernelGGL(sh::k_bp_delta0, dim3(1), dim3(64), 0, st, pcg->part_a, g, pcg->delta);
+                           pcg->s, pcg->x, nblk, zero_init ? 1 : 0, pcg->part_b);
+        // the sum by itself, where the host or the history needs it and no iteration follows
+        auto store_delta = [&](uint32_t it) {
+            hipLaunchKernelGGL(sh::k_bp_delta, dim3(1), dim3(64), 0, st, pcg->part_b, g, pcg->delta, it);
+        };
+        if (epsilon > 0.f || max_iterations == 0)
+            store_delta(0);
         if ((rc = sh::status_of(hipGetLastError())) != SH_OK)
             return rc;
         double delta0 = 0.0;
         if (epsilon > 0.f &&
             (rc = sh::status_of(hipMemcpyAsync(&delta0, pcg->delta, 8, hipMemcpyDeviceToHost, st))) != SH_OK)
             return rc;
-        float *r = pcg->r, *t = pcg->t;
+        // the built-in product takes the direction and the dot product into its
+        // kernel; any other operator needs the direction in memory
+        const sh_spmv *own = pcg->ops.apply_spmv == bcsr_apply_cb ? static_cast<const sh_spmv *>(pcg->ops.user) : nullptr;
+        if (own && own->rows != nblk)
+            own = nullptr;
+        float *r = pcg->r, *t = pcg->t, *d = pcg->d, *d_old = pcg->d_old;
         for (uint32_t it = 0; it < max_iterations; ++it)
         {
-            if ((rc = pcg->ops.apply_spmv(pcg->ops.user, pcg->d, pcg->q, stream)) != SH_OK)
-                return rc;
-            hipLaunchKernelGGL(sh::k_bp_dot, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->d, pcg->q, nblk,
-                               pcg->part_a);
-            hipLaunchKernelGGL(sh::k_bp_update, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->x, r, pcg->d, pcg->q,
-                               pcg->inv_diag, t, pcg->s, nblk, pcg->part_a, pcg->delta, it, pcg->part_b);
-            hipLaunchKernelGGL(sh::k_bp_dir, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->s, pcg->d, nblk,
-                               pcg->part_b, pcg->delta, it);
+            if (own)
+            {
+                hipLaunchKernelGGL(sh::k_bp_spmv, dim3(gq), dim3(sh::kBpSpmvThreads), 0, st, own->row_ptr, own->col,
+                                   own->blocks, pcg->s, d_old, d, pcg->q, nblk, pcg->part_b, g, pcg->delta, it,
+                                   pcg->part_a);
+            }
+            else
+            {
+                hipLaunchKernelGGL(sh::k_bp_dir, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->s, d, nblk, pcg->part_b,
+                                   pcg->delta, it);
+                if ((rc = sh::status_of(hipGetLastError())) != SH_OK ||
+                    (rc = pcg->ops.apply_spmv(pcg->ops.user, d, pcg->q, stream)) != SH_OK)
+                    return rc;
+                hipLaunchKernelGGL(sh::k_bp_dot, dim3(gq), dim3(sh::kBpSpmvThreads), 0, st, d, pcg->q, nblk, pcg->part_a);
+            }
+            hipLaunchKernelGGL(sh::k_bp_update, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->x, r, d, pcg->q,
+                               pcg->inv_diag, t, pcg->s, nblk, pcg->part_a, gq, pcg->delta, it, pcg->part_b);
+            if (epsilon > 0.f || it + 1 == max_iterations)
+                store_delta(it + 1);
             if ((rc = sh::status_of(hipGetLastError())) != SH_OK)
                 return rc;
             std::swap(r, t);
+            if (own)
+                std::swap(d, d_old);
             pcg->last_iters = it + 1;
             if (epsilon > 0.f)
             {

@@ -167,3 +167,62 @@ def test_block_pcg_converge_checked_and_errors(c1_system):
     bad_col[5] = N
     Abad = native.BlockCsr(_dev(torch, s["rp"]), _dev(torch, bad_col), _dev(torch, s["blk"]))
     assert Abad.check() == 1  # SH_E_ARG: a column out of range, found before any product reads it
+
+
+@pytest.mark.parametrize("rows,degree", [(1, 1), (2, 2), (7, 5), (11, 6), (41, 11), (40, 24), (300, 31), (8201, 4)])
+def test_block_csr_sizes(rows, degree):
+    """Rows that leave waves, work-groups and turns partly filled, rows of no
+    block, of one trip and of several: the product is the exact sum rounded
+    once (2^-24 of it, and an FP64 sum's own rounding), and the built-in
+    operator's fused iteration gives the callback's bits."""
+    import torch
+    from starhub_amd import native
+    torch.cuda.set_device(0)
+    rng = np.random.default_rng(rows)
+    cols = []
+    for r in range(rows):
+        near = rng.integers(0, rows, rng.integers(0, degree) if r % 5 else degree - 1)
+        cols.append(np.unique(np.concatenate([near, [r]])))
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.uint32)
+    col = np.concatenate(cols).astype(np.uint32)
+    blk = (rng.standard_normal((len(col), 6, 6)) * 0.02).astype(np.float32)
+    own = np.repeat(np.arange(rows), np.diff(rp)) == col
+    blk[own] = (0.5 * (blk[own] + blk[own].transpose(0, 2, 1)) + np.eye(6) * 3).astype(np.float32)
+    dinv = np.linalg.inv(blk[own].astype(np.float64)).astype(np.float32)
+    b = rng.standard_normal(6 * rows).astype(np.float32)
+    A = native.BlockCsr(_dev(torch, rp), _dev(torch, col), _dev(torch, blk.reshape(-1)))
+    assert A.check() == 0
+    v, y = _dev(torch, b), torch.full((6 * rows,), float("nan"), device="cuda")
+    assert A.apply(v.data_ptr(), y.data_ptr()) == 0
+    prod = blk.astype(np.float64) * b.reshape(-1, 6)[col][:, None, :]
+    exact, size = (np.zeros((rows, 6)) for _ in range(2))
+    np.add.at(exact, np.repeat(np.arange(rows), np.diff(rp)), prod.sum(2))
+    np.add.at(size, np.repeat(np.arange(rows), np.diff(rp)), np.abs(prod).sum(2))
+    torch.cuda.synchronize()
+    err = np.abs(y.cpu().numpy().reshape(-1, 6) - exact)
+    print("rows", rows, "blocks", len(col), "max err", err.max(), flush=True)
+    assert (err <= 2.0 ** -24 * np.abs(exact) + 2.0 ** -44 * size).all()
+
+    if rows > 1:  # the last row emptied
+        end = int(rp[-2])
+        rp2 = np.concatenate([rp[:-1], rp[-2:-1]])
+        cut = native.BlockCsr(_dev(torch, rp2), _dev(torch, col[:end]), _dev(torch, blk[:end].reshape(-1)))
+        y2 = torch.full_like(y, float("nan"))
+        assert cut.apply(v.data_ptr(), y2.data_ptr()) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y2[:-6], y[:-6]) and (y2[-6:] == 0).all()
+
+    @native.SPMV_APPLY_FN
+    def apply(user, xp, yp, stream):
+        return A.apply(xp, yp)
+
+    outs = []
+    for ops in (A.ops(), native.SpmvOps(None, 6 * rows, apply, native.SPMV_INIT_FN())):
+        pcg = native.BlockPCG(6 * rows)
+        x = torch.full((6 * rows,), 0.25, device="cuda")
+        assert pcg.set_input(_dev(torch, dinv), ops, v, x) == 0
+        pcg.solve(4, zero_init=False)
+        outs.append((x.cpu().numpy(), pcg.delta_history()))
+        pcg.close()
+    assert np.isfinite(outs[0][0]).all() and outs[0][1].shape == (5,)
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
