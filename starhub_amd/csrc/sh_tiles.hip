@@ -930,6 +930,7 @@ __global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__rest
     static_assert(kMatrixNodes * 68 <= kW, "one group's weights of the largest tile");
     __shared__ __align__(16) float Ht[kTileRec * kHStride]; // the records, a row per entry
     __shared__ __align__(16) float Ws[kW];                  // the weights, a row per node
+    __shared__ uint32_t odd[kGroups];                       // a group holds a record or weight that is not finite
     const int si = find_item(wg_begin, n_solve, blockIdx.x);
     const SolveDesc d = global_desc(sds[si]);
     const uint32_t t = blockIdx.x - wg_begin[si];
@@ -971,6 +972,7 @@ __global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__rest
     float w[K];
     uint32_t rank[2] = {0xffffffffu, 0xffffffffu};
     double cost = 0.0;
+    float probe = 0.f; // stays zero over finite values
     const uint32_t q = tid & 63u, grp = tid >> 6, col = (q & 3u) * 16u + (q >> 2); // of the thread's pixel
     if (tid < np)
     {
@@ -985,16 +987,28 @@ __global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__rest
             load_hg<JT>(d.jr, p, hg);
 #pragma unroll
         for (int e = 0; e < kTileRec; ++e)
+        {
             Ht[uint32_t(e) * kHStride + grp * 64u + col] = hg[e];
+            probe = fmaf(hg[e], 0.f, probe);
+        }
         w[0] = wa.x, w[1] = wa.y, w[2] = wa.z, w[3] = wa.w;
         w[4] = wb.x, w[5] = wb.y, w[6] = wb.z, w[7] = wb.w;
         rank[0] = rk.x;
         rank[1] = rk.y;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            probe = fmaf(w[k], 0.f, probe);
     }
     else if (tid < uint32_t(TP))
 #pragma unroll
         for (int e = 0; e < kTileRec; ++e)
             Ht[uint32_t(e) * kHStride + grp * 64u + col] = 0.f;
+    if (tid < uint32_t(TP))
+    {
+        const bool any = __any(!(probe == 0.f));
+        if (lane == 0)
+            odd[grp] = any;
+    }
     if constexpr (FUSED)
     {
         // the cost partials of the tile's 64-pixel groups, as the term kernel writes them
@@ -1026,7 +1040,29 @@ __global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__rest
         const uint32_t g = whole ? wave >> 1 : g0;
         if (g0)
             group_at(g);
-        if (m < se)
+        if (odd[g])
+        {
+            // a product with a zero weight would spread infinities and NaN to
+            // pairs the pixel does not name: the slots one by one instead
+            for (; m < se; m += 16u * step)
+                for (uint32_t s = m; s < min(m + 16u, se); ++s)
+                {
+                    const uint32_t nodes = d.slot_pair[s0 + s];
+                    const float *wa = Ws + (nodes & 255u) * wstride + (g - g0) * 64u;
+                    const float *wb = Ws + (nodes >> 8) * wstride + (g - g0) * 64u;
+                    float acc = 0.f;
+                    if (lane < uint32_t(kTileRec))
+                        for (uint32_t i = 0; i < 64u; ++i)
+                        {
+                            const uint32_t ci = (i & 3u) * 16u + (i >> 2);
+                            if (wa[ci] != 0.f && wb[ci] != 0.f)
+                                acc = fmaf(wa[ci] * wb[ci], Ht[lane * kHStride + g * 64u + ci], acc);
+                        }
+                    if (lane < 32u)
+                        out[size_t(d.slot_pos[s0 + s]) * kPartStride + lane] = acc;
+                }
+        }
+        else if (m < se)
         {
             v4f h0[4], h1[4]; // records: entries c and 16 + c
 #pragma unroll

@@ -35,7 +35,7 @@ def test_tiles_by_node_count(tile_pix, fp16):
             knn[s] = x0 + rng.choice(size, K, replace=False)
     prod = dict(prod, surfel_knn=knn.reshape(prod["surfel_knn"].shape))
 
-    def solve(flags):
+    def solve(flags, prod=prod):
         s = native.WarpSolver(native.make_config(cfg.solver, cfg.width, cfg.height, N, K, flags=flags))
         f, _ = workload.device_frame(sc, producers=prod)
         s.process_frame(f)
@@ -50,3 +50,18 @@ def test_tiles_by_node_count(tile_pix, fp16):
         # the same products of the same records in FP32, in another order: 168
         # roundings of 2^-24 of the largest entry, all one way, reach 1e-5
         assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+
+    # a weight that is not finite reaches the blocks and rows of its node's
+    # pixels, and no others: the same entries as in the other path
+    weights = prod["surfel_spatial"].reshape(-1, K).copy()
+    row = idx[100][idx[100] != 0xFFFFFFFF]
+    weights[row[::40], 2] = np.inf
+    odd = dict(prod, surfel_spatial=weights.reshape(prod["surfel_spatial"].shape))
+    split = native.SH_FLAG_NO_PERSISTENT_PCG  # its solve ends without exchanging what is not finite
+    tiled, rows = solve(flag | split, odd), solve(native.SH_FLAG_ROW_SEGMENTS | split, odd)
+    for name in ("blk", "rhs"):
+        a, b = tiled[name], rows[name]
+        fin = np.isfinite(b)
+        print(tile_pix, fp16, name, "finite", fin.sum(), "of", fin.size, flush=True)
+        assert 0 < fin.sum() < fin.size and np.array_equal(fin, np.isfinite(a))
+        assert np.abs(a[fin] - b[fin]).max() <= 1e-5 * np.abs(b[fin]).max()
