@@ -138,7 +138,7 @@ def solve_bytes(cfg, P: int, U: int) -> float:
 
 KERNEL_OF_PHASE = {"dense_terms": "k_terms", "reg_terms": "k_terms", "rows_seg": "k_rows_seg",
                    "rows_combine": "k_rows_combine", "dinv": "k_dinv", "pcg": "k_pcg_resident",
-                   "update": "k_update", "tiles": "k_tiles", "tiles_combine": "k_tiles_combine"}
+                   "update": "k_update", "tiles": "k_tiles_matrix", "tiles_combine": "k_tiles_combine"}
 
 
 def pcg_kernel(tuning: dict) -> str:
