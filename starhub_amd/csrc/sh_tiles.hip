@@ -1043,21 +1043,33 @@ __global__ __launch_bounds__(2 * TP) void k_tiles_matrix(const SolveDesc *__rest
         if (odd[g])
         {
             // a product with a zero weight would spread infinities and NaN to
-            // pairs the pixel does not name: the slots one by one instead
+            // pairs the pixel does not name: the slots one by one instead, each
+            // over the pixels that name both of its nodes (by the ranks: a node
+            // may be named with weight zero).  Lane i answers for pixel i.
+            uint2 rk = make_uint2(0xffffffffu, 0xffffffffu);
+            if (g * 64u + lane < np)
+                rk = reinterpret_cast<const uint2 *>(d.gprank)[p0 + g * 64u + lane];
+            auto names = [&](uint32_t r) {
+                bool is = false;
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    is = is || (((k < 4 ? rk.x : rk.y) >> (8 * (k & 3))) & 255u) == r;
+                return is;
+            };
             for (; m < se; m += 16u * step)
                 for (uint32_t s = m; s < min(m + 16u, se); ++s)
                 {
                     const uint32_t nodes = d.slot_pair[s0 + s];
                     const float *wa = Ws + (nodes & 255u) * wstride + (g - g0) * 64u;
                     const float *wb = Ws + (nodes >> 8) * wstride + (g - g0) * 64u;
+                    unsigned long long px = __ballot(names(nodes & 255u) && names(nodes >> 8));
                     float acc = 0.f;
-                    if (lane < uint32_t(kTileRec))
-                        for (uint32_t i = 0; i < 64u; ++i)
-                        {
-                            const uint32_t ci = (i & 3u) * 16u + (i >> 2);
-                            if (wa[ci] != 0.f && wb[ci] != 0.f)
-                                acc = fmaf(wa[ci] * wb[ci], Ht[lane * kHStride + g * 64u + ci], acc);
-                        }
+                    for (; px; px &= px - 1)
+                    {
+                        const uint32_t i = uint32_t(__ffsll(px)) - 1u, ci = (i & 3u) * 16u + (i >> 2);
+                        if (lane < uint32_t(kTileRec))
+                            acc = fmaf(wa[ci] * wb[ci], Ht[lane * kHStride + g * 64u + ci], acc);
+                    }
                     if (lane < 32u)
                         out[size_t(d.slot_pos[s0 + s]) * kPartStride + lane] = acc;
                 }

@@ -65,3 +65,62 @@ def test_tiles_by_node_count(tile_pix, fp16):
         print(tile_pix, fp16, name, "finite", fin.sum(), "of", fin.size, flush=True)
         assert 0 < fin.sum() < fin.size and np.array_equal(fin, np.isfinite(a))
         assert np.abs(a[fin] - b[fin]).max() <= 1e-5 * np.abs(b[fin]).max()
+
+
+def _chains(tile_pix, size, fp16=False):
+    """A frame whose full tiles name exactly `size` nodes each: the p-th pixel of the tile order names eight nodes in a
+    row, the first of them p mod (size - 7), so any size - 7 pixels in a row name all of them, in at most 484 pairs of
+    64 nodes.  Returns a solver of it by (flags, producers, scene), its scene and producers, and the pixel order."""
+    import torch
+    from starhub_amd import native, scene, workload
+    torch.cuda.set_device(0)
+    base = scene.config_c2()
+    cfg = replace(base, num_surfels=60000, num_nodes=200, width=331, height=203, fx=290.0, fy=290.0, with_flow=False,
+                  solver=replace(base.solver, gn_iterations=1, fp16=fp16))
+    sc = scene.generate(cfg)
+    there = sc.index_map != 0xFFFFFFFF
+    index = sc.index_map.copy()
+    index[there] = np.arange(there.sum())  # a surfel of its own for every pixel
+    sc = replace(sc, index_map=index)
+    _, prod = workload.device_frame(sc)
+
+    def solve(flags, prod, scn=sc, names=("blk", "rhs")):
+        s = native.WarpSolver(native.make_config(cfg.solver, cfg.width, cfg.height, cfg.num_nodes, cfg.K, flags=flags))
+        s.process_frame(workload.device_frame(scn, producers=prod)[0])
+        out = {n: s.debug(n, torch.int16 if n == "gpix" else torch.int32 if n == "tile_nodes" else torch.float32)
+               .cpu().numpy() for n in names}
+        s.close()
+        return out
+
+    flag = {64: native.SH_FLAG_TILE_PIX_64, 128: 0, 256: native.SH_FLAG_TILE_PIX_256}[tile_pix]
+    pix = solve(flag, prod, names=("gpix",))["gpix"].view(np.uint16).reshape(-1, 4).astype(np.int64)
+    knn = prod["surfel_knn"].reshape(-1, cfg.K).copy()
+    knn[index[pix[:, 1], pix[:, 0]]] = (np.arange(len(pix)) % (size - 7))[:, None] + np.arange(cfg.K)
+    return solve, sc, dict(prod, surfel_knn=knn.reshape(prod["surfel_knn"].shape)), pix, flag
+
+
+@pytest.mark.parametrize("size", [8, 32, 33, 64, 65])
+@pytest.mark.parametrize("tile_pix", [64, 128, 256])
+def test_tiles_record_not_finite(tile_pix, size):
+    """A measured normal that is NaN makes its pixel's record NaN, and so every block of two nodes that the pixel
+    names, a node of weight zero too (0 x NaN), and no other block: the same entries as in the pair-major path."""
+    from starhub_amd import native
+    solve, sc, prod, pix, flag = _chains(tile_pix, size)
+    normal = sc.measure_normal.copy()
+    weights = prod["surfel_spatial"].reshape(-1, 8).copy()
+    for p, slot in ((2 * len(pix) // 3, 2), (len(pix) - 3, 5)):  # one of them in the last, partial tile
+        x, y, tx, ty = pix[p]
+        normal[ty, tx, :3] = np.nan
+        weights[sc.index_map[y, x], slot] = 0.0
+    prod = dict(prod, surfel_spatial=weights.reshape(prod["surfel_spatial"].shape))
+    odd = replace(sc, measure_normal=normal)
+    split = native.SH_FLAG_NO_PERSISTENT_PCG  # its solve ends without exchanging what is not finite
+    tiled, pairs = solve(flag | split, prod, odd), solve(native.SH_FLAG_PAIR_MAJOR | split, prod, odd)
+    for name in ("blk", "rhs"):
+        a, b = tiled[name], pairs[name]
+        fin = np.isfinite(b)
+        print(tile_pix, size, name, "finite", fin.sum(), "of", fin.size, "differ", (fin != np.isfinite(a)).sum(), flush=True)
+        assert 0 < fin.sum() < fin.size and np.array_equal(fin, np.isfinite(a))
+        # as in test_tiles_by_node_count, for the sums of more pixels: the
+        # products of a block's up to P / (size - 7) pixels in another order
+        assert np.abs(a[fin] - b[fin]).max() <= 2.0 ** -24 * (len(pix) // (size - 7) + 8) * np.abs(b[fin]).max()
