@@ -47,13 +47,11 @@ __device__ __forceinline__ uint32_t c_ka(uint32_t c) { return (c >> kPixBits) & 
 __device__ __forceinline__ uint32_t c_kb(uint32_t c) { return (c >> (kPixBits + 3)) & 7u; }
 // A slot is a block's contributions from one group of kSlotPix consecutive
 // pixels of a tile, so a slot's list is at most kSlotPix long and k_tiles'
-// longest serial sum is bounded.
-#ifndef SH_SLOT_SHIFT
-#define SH_SLOT_SHIFT 6
-#endif
-constexpr int kSlotShift = SH_SLOT_SHIFT;
+// longest serial sum is bounded.  k_tiles_matrix sums a slot over a whole
+// group, a lane a pixel.
+constexpr int kSlotShift = 6;
 constexpr int kSlotPix = 1 << kSlotShift;
-static_assert((1 << kSlotShift) == kSlotPix && kSlotPix >= 32, "slot pixel groups");
+static_assert(kSlotPix == 64 && kTileGroups * kSlotPix == kTilePixMax, "a slot's pixel group is a wave of pixels");
 
 // A tile of TP pixels for K nodes per pixel: two threads per pixel.
 template <int K, int TP>
@@ -607,8 +605,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_compact(IndexGroup g, con
             const uint32_t c = src[ws.tslot_first[tbase + s]];
             const uint8_t *__restrict__ rk = d.gprank + (size_t(t) * TP + c_pix(c)) * K;
             d.slot_pair[s0 + s] = uint16_t(rk[c_ka(c)] | (uint32_t(rk[c_kb(c)]) << 8));
-            const uint32_t g1 = c_pix(c) >> 6;
-            const uint32_t first = s == 0 ? 0u : (c_pix(src[ws.tslot_first[tbase + s - 1]]) >> 6) + 1u;
+            const uint32_t g1 = c_pix(c) >> kSlotShift;
+            const uint32_t first = s == 0 ? 0u : (c_pix(src[ws.tslot_first[tbase + s - 1]]) >> kSlotShift) + 1u;
             for (uint32_t gr = first; gr <= g1; ++gr)
                 tg[gr] = uint16_t(s);
             if (s + 1 == ns)
