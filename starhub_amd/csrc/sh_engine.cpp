@@ -181,9 +181,6 @@ int Engine::init(const sh_solver_config &c, uint32_t max_slots)
         A(d.seg_ptr, size_t(ncap_ + 1) * 4);
         A(d.tile_cbase, size_t(div_up(pcap_, kTilePixMin) + 1) * 4);
         A(d.tile_sbase, size_t(div_up(pcap_, kTilePixMin) + 1) * 4);
-        A(d.tile_nodes, size_t(div_up(pcap_, kTilePixMin)) * 4);
-        A(d.tile_group, size_t(div_up(pcap_, kTilePixMin)) * (kTileGroups + 1) * 2);
-        A(d.gprank, size_t(pcap_) * K_);
         A(d.list_off, (size_t(ncap_) + 2 * size_t(ucap_) + 1) * 4);
         A(d.blk_transpose, (size_t(ncap_) + 2 * size_t(ucap_)) * 4);
         A(d.jr, size_t(pcap_) * kHG * (fp16_ ? 2 : 4));
@@ -225,6 +222,18 @@ int Engine::init(const sh_solver_config &c, uint32_t max_slots)
     A(d_slots_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot));
     A(d_slots2_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot2));
     A(d_flags_, 64);
+    // The resident PCG's groups wait for each other through d_slots_, and how
+    // long depends on which 4 KB page of memory that is: a solve of 200 nodes
+    // takes 806 to 866 us with only that page changed (pages two apart differ
+    // by 25 to 55 us, neighbouring pairs agree), and the allocations before it
+    // decide.  So arrays that the exchange does not use are allocated behind it.
+    for (Slot &sl : slots_)
+    {
+        SolveDesc &d = sl.d;
+        A(d.tile_nodes, size_t(tiles_cap_) * 4);
+        A(d.tile_group, size_t(tiles_cap_) * (kTileGroups + 1) * 2);
+        A(d.gprank, size_t(pcap_) * K_);
+    }
     SH_HIP(hipMemset(d_slots_, 0, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot)));
     SH_HIP(hipMemset(d_slots2_, 0, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot2)));
     SH_HIP(hipMemset(d_flags_, 0, 64));
