@@ -74,7 +74,7 @@ struct SolveDesc
     int tile_pix;            // pixels per tile (64, 128 or 256) of the index build
     uint32_t *tile_cbase;    // n_tiles+1: first contribution of each tile
     uint32_t *tile_sbase;    // n_tiles+1: first slot of each tile
-    uint32_t *tile_nodes;    // n_tiles: distinct nodes of each tile (above kMatrixNodes: its slots are summed from lists)
+    uint32_t *tile_nodes;    // n_tiles: distinct nodes of each tile (above kMatrixNodes: only the list form sums its slots)
     uint8_t *gprank;         // P*K: each pixel slot's node as its rank in the tile (kNoRank: a later slot names it too)
     uint16_t *tile_group;    // n_tiles*(kTileGroups+1): first slot of each 64-pixel group of a tile, then their end
     uint16_t *slot_pair;     // S: the ranks of a slot's nodes, ra | rb << 8

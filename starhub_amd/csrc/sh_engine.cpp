@@ -1711,6 +1711,7 @@ int Engine::debug_view(uint32_t slot, const char *name, const void **ptr, size_t
         {"seg_ptr", d.seg_ptr, N + 1},
         {"tile_cbase", d.tile_cbase, size_t(d.n_tiles) + 1},
         {"tile_sbase", d.tile_sbase, size_t(d.n_tiles) + 1},
+        {"tile_nodes", d.tile_nodes, size_t(d.n_tiles)},
         {"list_off", d.list_off, N + 2 * U + 1},
         {"blk_transpose", d.blk_transpose, N + 2 * U},
         {"reg", d.reg, E * kReg},

@@ -111,7 +111,7 @@ private:
         float *tpw = nullptr;
         uint32_t max_row_len = 0;
         uint32_t tile_slot_max = 0; // largest slot count of one tile
-        uint32_t tiles_listed = 0; // tiles of the last index build above kMatrixNodes
+        uint32_t tiles_listed = 0; // tiles of the last index build that only the list form sums
         bool records_fused = false;  // the last GN iteration built its records in the tile kernel (not stored)
         void *part_buf = nullptr; // segment partials, grown on demand
         size_t part_bytes = 0;

@@ -47,7 +47,7 @@ struct IndexWs
     uint32_t *flags, *pos;         // raster valid flags and their exclusive scan
     uint32_t *tflags, *tpos;       // the same in tile order
     uint32_t *errs;                // one range-check word per item
-    uint32_t *meta;                // 16 words per item: [0] longest row, [kMetaListed] tiles above kMatrixNodes
+    uint32_t *meta;                // 16 words per item: [0] longest row, [kMetaListed] tiles only the list form sums
     uint32_t *bitmap;              // kBitmapWords per node key
     uint2 *bitpre;                 // the same words with the neighbour count of the words before each
     uint32_t *rowlen, *segcnt;     // per node key
@@ -88,7 +88,7 @@ hipError_t launch_scan_jobs(const ScanJob *jobs, uint32_t n_jobs, hipStream_t st
 // Counts for the host, host[item * 8 + k]: stage 1 -> [0] valid pixels,
 // [1] range-check flag (then cleared); stage 2 -> [0] segments, [1] longest
 // row, [2] U, [3] slots, [4] contributions, [5] largest tile slot count,
-// [6] tiles with more than kMatrixNodes nodes.
+// [6] tiles that only the list form sums.
 hipError_t launch_index_counts(const IndexGroup &g, int stage, const IndexWs &ws, uint32_t *host, hipStream_t st);
 hipError_t launch_pair_kv(const SolveDesc &d, uint32_t *keys, uint32_t *vals, hipStream_t st);
 hipError_t launch_pair_heads(const uint32_t *keys, uint32_t n, uint32_t *head, uint32_t *meta, hipStream_t st);
@@ -268,7 +268,8 @@ hipError_t launch_block_transpose(const IndexGroup &g, const uint32_t *wmap, uin
 // fused: the tile kernel builds the FP32 per-pixel records itself (and the
 // dense cost partials) from the warp field of GN iteration offset parity,
 // instead of reading them; the term kernel then runs the ARAP part only.
-// n_listed: tiles of the launch with more than kMatrixNodes nodes.
+// n_listed (at most n_wg): tiles of the launch that only the list form sums
+// (more than kMatrixNodes nodes, or too many pairs).
 hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int parity, const SolveDesc *sds,
                         const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, uint32_t n_listed,
                         hipStream_t st);

@@ -655,7 +655,7 @@ __global__ __launch_bounds__(kTileThreads) void k_block_transpose(IndexGroup g, 
 template <int K, class JT, int TP, bool FUSED>
 __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ sds,
                                                         const uint32_t *__restrict__ wg_begin, int n_solve,
-                                                        uint32_t slot_cap, int parity)
+                                                        uint32_t slot_cap, int parity, bool all)
 {
     using G = TileGeom<K, TP>;
     constexpr int NT = G::kThreads;
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ 
     const uint32_t t = blockIdx.x - wg_begin[si];
     if (t >= uint32_t(d.n_tiles))
         return; // uniform over the group
-    if (K == 8 && d.tile_nodes[t] <= kMatrixNodes)
+    if (K == 8 && !all && d.tile_nodes[t] <= kMatrixNodes)
         return; // k_tiles_matrix sums this tile
     const uint32_t tid = threadIdx.x;
     const uint32_t p0 = t * TP;
@@ -906,7 +906,8 @@ __global__ __launch_bounds__(2 * TP) void k_tiles(const SolveDesc *__restrict__ 
 // v_mfma_f32_16x16x4_f32 adds its four products one after another, each fused
 // and rounded as fmaf, so over pixels in order (and zeros in between) a slot
 // has the list form's sum, bit for bit.
-// For K = 4 a pixel has ten pairs, not 36, and the lists are the better form.
+// For K = 4 a pixel has ten pairs, not 36, and the lists are the better form;
+// launch_tiles has the rule for launches that need both.
 // Twelve solves of 128 to 4096 nodes: 186 us a launch from the lists, 147 us
 // so; 640x480 24.5 and 19.8 us; 1280x720 with FP16 records 44 and 33 us.  What
 // bounds it now is the chain of loads in front of a tile's records (work map,
@@ -2191,6 +2192,17 @@ hipError_t launch_block_transpose(const IndexGroup &g, const uint32_t *wmap, uin
     return hipGetLastError();
 }
 
+// A launch of K = 8 with tiles that only the list form sums (n_listed of them)
+// takes the matrix form for its other tiles when these hold at least this many
+// pixels, and the list form for all its tiles otherwise.  Per tile the matrix
+// form takes 0.79 of the list form's time, but the second launch takes at
+// least a tile's latency, about 17 us.  Solves (six iterations) of one frame
+// with 59 listed tiles and one, two, three, six or twelve with none (1780,
+// 3339, 4699, 7763 and 10535 128-pixel tiles): 2600, 2875, 2885, 3711 and 4390
+// us with both forms, 2540, 2879, 2929, 3760 and 4541 us from the lists; one of
+// 232 tiles, some of them listed: 2595 and 2388 us.
+constexpr uint64_t kTwoFormPixels = 512 * 1024;
+
 hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int parity, const SolveDesc *sds,
                         const uint32_t *wmap, int n_solve, uint32_t n_wg, uint32_t slot_cap, uint32_t n_listed,
                         hipStream_t st)
@@ -2204,7 +2216,9 @@ hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int par
     return with_tile_pix(tile_pix, [&](auto tp) {
         constexpr int TP = decltype(tp)::value;
         const dim3 grid(n_wg), block(2 * TP);
-        if (K == 8)
+        const bool matrix =
+            K == 8 && (n_listed == 0 || uint64_t(n_wg - n_listed) * uint64_t(TP) >= kTwoFormPixels);
+        if (matrix)
         {
             if (fused)
                 hipLaunchKernelGGL((k_tiles_matrix<float, TP, true>), grid, block, 0, st, sds, wmap, n_solve, parity);
@@ -2216,25 +2230,26 @@ hipError_t launch_tiles(int K, bool fp16, uint32_t tile_pix, bool fused, int par
                                    parity);
             if (n_listed == 0)
                 return;
-            if (fused)
-                hipLaunchKernelGGL((k_tiles<8, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                                   parity);
-            else if (fp16)
-                hipLaunchKernelGGL((k_tiles<8, __half, TP, false>), grid, block, lds, st, sds, wmap, n_solve,
-                                   slot_cap, parity);
-            else
-                hipLaunchKernelGGL((k_tiles<8, float, TP, false>), grid, block, lds, st, sds, wmap, n_solve,
-                                   slot_cap, parity);
         }
+        const bool all = !matrix;
+        if (K == 8 && fused)
+            hipLaunchKernelGGL((k_tiles<8, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
+                               parity, all);
+        else if (K == 8 && fp16)
+            hipLaunchKernelGGL((k_tiles<8, __half, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
+                               parity, all);
+        else if (K == 8)
+            hipLaunchKernelGGL((k_tiles<8, float, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
+                               parity, all);
         else if (fused)
             hipLaunchKernelGGL((k_tiles<4, float, TP, true>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
+                               parity, all);
         else if (fp16)
             hipLaunchKernelGGL((k_tiles<4, __half, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
+                               parity, all);
         else
             hipLaunchKernelGGL((k_tiles<4, float, TP, false>), grid, block, lds, st, sds, wmap, n_solve, slot_cap,
-                               parity);
+                               parity, all);
     });
 }
 

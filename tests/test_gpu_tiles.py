@@ -1,6 +1,6 @@
-"""The tile kernel's matrix form against the row-segment path (no tiles), by the number of distinct nodes a tile
-names: up to 32 (a tile's weights whole), 33 to 64 (a group at a time), more (the list form, in the same launch), for
-every tile size, FP32 and FP16 records, and a last tile of a few pixels."""
+"""The tile kernel against paths without tiles, for every tile size, FP32 and FP16 records and a last tile of a few
+pixels: the matrix form with tiles of up to 32 distinct nodes (their weights whole) and of 33 to 64 (a group at a time),
+the list form, which sums every tile of a small launch that holds one of more nodes or pairs, and a launch of both."""
 from dataclasses import replace
 
 import numpy as np
@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("fp16", [False, True])
 @pytest.mark.parametrize("tile_pix", [64, 128, 256])
 def test_tiles_by_node_count(tile_pix, fp16):
+    """Tiles of 8 to 100 nodes and many pairs in one frame, so the list form and both ways its index is built."""
     import torch
     from starhub_amd import native, scene, workload
     assert torch.cuda.is_available()
@@ -97,6 +98,52 @@ def _chains(tile_pix, size, fp16=False):
     knn = prod["surfel_knn"].reshape(-1, cfg.K).copy()
     knn[index[pix[:, 1], pix[:, 0]]] = (np.arange(len(pix)) % (size - 7))[:, None] + np.arange(cfg.K)
     return solve, sc, dict(prod, surfel_knn=knn.reshape(prod["surfel_knn"].shape)), pix, flag
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("size", [8, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("tile_pix", [64, 128, 256])
+def test_tiles_of_exact_node_counts(tile_pix, size, fp16):
+    """The matrix form on both sides of its limits of 32 and 64 nodes (65: the list form), by the counts the index
+    found."""
+    from starhub_amd import native
+    solve, _, prod, pix, flag = _chains(tile_pix, size, fp16)
+    tiled = solve(flag, prod, names=("blk", "rhs", "tile_nodes"))
+    nodes, full = tiled["tile_nodes"], len(pix) // tile_pix
+    assert len(nodes) == -(-len(pix) // tile_pix) and (nodes[:full] == size).all() and (nodes <= size).all()
+    rows = solve(native.SH_FLAG_ROW_SEGMENTS, prod)
+    for name in ("blk", "rhs"):
+        a, b = tiled[name], rows[name]
+        print(tile_pix, size, fp16, name, "max diff", np.abs(a - b).max(), "max", np.abs(b).max(), flush=True)
+        # a block's products of up to len(pix) / (size - 7) pixels in another order
+        assert np.abs(a - b).max() <= 2.0 ** -24 * (len(pix) // (size - 7) + 8) * np.abs(b).max()
+
+
+def test_both_tile_forms_in_a_launch():
+    """Frames of 33-node tiles, enough pixels for a launch of their own, and one of 65-node tiles, which the list form
+    sums: every solve has the bits it has alone."""
+    import torch
+    from starhub_amd import native, workload
+    _, sc, prod, pix, _ = _chains(128, 33)
+    _, sc2, prod2, _, _ = _chains(128, 65)
+    n = 512 * 1024 // (len(pix) // 128 * 128) + 2
+    frame, other = workload.device_frame(sc, producers=prod)[0], workload.device_frame(sc2, producers=prod2)[0]
+    cfg, split = sc.cfg, native.SH_FLAG_NO_PERSISTENT_PCG
+    conf = native.make_config(cfg.solver, cfg.width, cfg.height, cfg.num_nodes, cfg.K, flags=split)
+    batch = native.BatchSolver(conf, n)
+    for i in range(n):
+        batch.set_inputs(i, other if i == 5 else frame)
+    batch.solve(n)
+    alone = []
+    for f in (frame, other):
+        s = native.WarpSolver(conf)
+        s.process_frame(f)
+        alone.append(s.node_se3())
+        s.close()
+    assert bool(torch.isfinite(alone[0]).all()) and not torch.equal(alone[0], alone[1])
+    for i in range(n):
+        assert torch.equal(batch.node_se3(i), alone[i == 5]), i
+    batch.close()
 
 
 @pytest.mark.parametrize("size", [8, 32, 33, 64, 65])
