@@ -10,16 +10,16 @@
 //
 // Once per solve (index build), one work-group per tile lists the tile's
 // contributions -- (node pair (a <= b) of distinct nodes of a pixel, pixel,
-// slot of a, slot of b) -- in (upper block of the pair, pixel) order: by the
+// slot of a, slot of b) -- slot by slot, a slot's in pixel order: by the
 // ranks of its node pairs and a pixel mask per pair (or, for a tile with
-// too many nodes, an LDS radix sort of the keys).  Equal blocks within a
-// group of kSlotPix pixels form a slot; slots are numbered across tiles in
-// tile order, and a stable sort of the slots by block gives every block the
-// list of its slot partials in tile order.
+// too many nodes or pairs, an LDS radix sort of the keys).  Equal blocks
+// within a group of kSlotPix pixels form a slot; slots are numbered across
+// tiles in tile order, and a stable sort of the slots by block gives every
+// block the list of its slot partials in tile and group order.
 //
-// Per GN iteration, one work-group per tile stages its records, weights and
-// contribution list in LDS and sums every slot's contributions in pixel
-// order (w_a w_b H, and w_a^2 g on diagonal slots); the combine kernel adds a
+// Per GN iteration, one work-group per tile sums every slot's contributions in
+// pixel order (w_a w_b H, and w_a^2 g on diagonal slots), as a matrix product
+// or from the list; the combine kernel adds a
 // block's slot partials in list order, the row's ARAP and node-translation
 // terms and the damping.  Each record is read once per GN iteration, there
 // are no atomics, and every sum has a fixed order.
@@ -187,7 +187,9 @@ struct TileRankLds
     uint32_t total[2];
 };
 
-// Per tile: the contributions in block order, each block's in pixel order,
+// Per tile: the contributions group of kSlotPix pixels by group, in each in
+// block order and each block's in pixel order (the sorting path below: block
+// by block, each block's in pixel order, so that a slot's are together too),
 // at the tile's fixed stride in the workspace: the packed contributions
 // (pixel | ka << 8 | kb << 11), each slot's block and first contribution (a
 // slot: the contributions of one block and one group of kSlotPix pixels),
@@ -200,7 +202,11 @@ struct TileRankLds
 // A tile with more nodes or pairs than that LDS holds sorts its
 // (block << 8 | pixel) keys instead (a stable LDS radix sort).  Compiled for
 // five 128-pixel tiles a CU (at most 102 registers; the kernel waits mostly
-// on memory and barriers, so more tiles in flight pay).
+// on memory and barriers, so more tiles in flight pay).  What a pair's item
+// number says (its slots) is not kept, and the node ids are not kept past
+// the pairs: with both in registers across the ranking it took 43.8 us at
+// 640x480 and 28.5 us at 320x240, 31.9 and 17.5 us so (128-pixel tiles,
+// K = 8); the sorting path alone still spills.
 template <int K, int TP>
 __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup g, const uint32_t *__restrict__ wmap,
                                                                       IndexWs ws)
@@ -241,15 +247,17 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
     uint16_t *__restrict__ cout = ws.tcontrib + tbase;
 
     // this thread's half of the pixel's pairs: q = i or kItems + i, as
-    // (lo | hi << 16) and (ka | kb << 3); all ones: no contribution
+    // (lo | hi << 16), all ones: no contribution; its slots as (ka | kb << 3)
+    // follow from i
     uint32_t lohi[G::kItems];
-    uint8_t vals[G::kItems];
 #pragma unroll
     for (int i = 0; i < G::kItems; ++i)
-    {
         lohi[i] = 0xffffffffu;
-        vals[i] = 0;
-    }
+    auto slots_of = [half](int i) __attribute__((always_inline)) { // folds to a select of two constants
+        const int q0 = pair_first<K>(i) | (pair_second<K>(i) << 3);
+        const int q1 = pair_first<K>(G::kItems + i) | (pair_second<K>(G::kItems + i) << 3);
+        return uint32_t(half ? q1 : q0);
+    };
     uint16_t kn[K];
     bool act[K];
 #pragma unroll
@@ -279,10 +287,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
             const bool on_a = half ? act[ka1] : act[ka0], on_b = half ? act[kb1] : act[kb0];
             const uint32_t na = half ? kn[ka1] : kn[ka0], nb = half ? kn[kb1] : kn[kb0];
             if (on_a && on_b)
-            {
                 lohi[i] = min(na, nb) | (max(na, nb) << 16);
-                vals[i] = uint8_t(half ? (ka1 | (kb1 << 3)) : (ka0 | (kb0 << 3)));
-            }
         }
     }
 
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
     __syncthreads();
     const uint32_t dn = r.total[0];
     bool ranked = dn <= uint32_t(R::kMaxNodes);
-    uint32_t pk[G::kItems]; // pair keys, then pair ranks
+    uint32_t pk[G::kItems]; // pair keys, then pair ranks (all ones: no contribution)
     if (ranked)
     {
         const uint32_t pwords = (dn * dn + 31u) / 32u;
@@ -338,27 +343,37 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
         auto nrank = [&](uint32_t n) {
             return uint32_t(r.npre[n >> 5]) + uint32_t(__popc(r.nbits[n >> 5] & ((1u << (n & 31u)) - 1u)));
         };
-        // the pixel's nodes as ranks, half of them per thread (K = 8)
-        if constexpr (K == 8)
-            if (p < uint32_t(d.P))
-            {
-                uint32_t ranks = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                {
-                    const bool on = half ? act[j + 4] : act[j];
-                    const uint32_t n = half ? kn[j + 4] : kn[j];
-                    ranks |= (on ? nrank(n) : kNoRank) << (8 * j);
-                }
-                reinterpret_cast<uint32_t *>(d.gprank)[size_t(p) * 2 + half] = ranks;
-            }
+        // and the ranks of the pixel's nodes (K = 8), from the pairs of a node
+        // with itself: bytes 0 .. 2 from the pixel's first thread, 3 .. 7 from
+        // its second
+        uint32_t ranks[2] = {0u, 0u};
 #pragma unroll
         for (int i = 0; i < G::kItems; ++i)
+        {
+            pk[i] = 0xffffffffu;
+            uint32_t ra = kNoRank;
             if (lohi[i] != 0xffffffffu)
             {
-                pk[i] = nrank(lohi[i] & 0xffffu) * dn + nrank(lohi[i] >> 16);
+                ra = nrank(lohi[i] & 0xffffu);
+                pk[i] = ra * dn + nrank(lohi[i] >> 16);
                 atomicOr(&r.pbits[pk[i] >> 5], 1u << (pk[i] & 31u));
             }
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+            {
+                const int own = pair_first<K>(i) == k && pair_second<K>(i) == k ? 0
+                                : pair_first<K>(G::kItems + i) == k && pair_second<K>(G::kItems + i) == k ? 1
+                                                                                                          : 2;
+                if (own < 2)
+                    ranks[k >> 2] |= half == uint32_t(own) ? ra << (8 * (k & 3)) : 0u;
+            }
+        }
+        if constexpr (K == 8)
+        {
+            const uint32_t r0 = ranks[0] | __shfl_xor(ranks[0], 1, 64), r1 = ranks[1] | __shfl_xor(ranks[1], 1, 64);
+            if (p < uint32_t(d.P))
+                reinterpret_cast<uint32_t *>(d.gprank)[size_t(p) * 2 + half] = half ? r1 : r0;
+        }
         __syncthreads();
         // pair ranks: exclusive prefix of the word popcounts, a run of words per thread
         const uint32_t per = (pwords + G::kThreads - 1) / G::kThreads;
@@ -383,7 +398,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < G::kItems; ++i)
-                if (lohi[i] != 0xffffffffu)
+                if (pk[i] != 0xffffffffu)
                 {
                     const uint32_t key = pk[i];
                     pk[i] = uint32_t(r.ppre[key >> 5]) + uint32_t(__popc(r.pbits[key >> 5] & ((1u << (key & 31u)) - 1u)));
@@ -444,7 +459,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
             // each contribution at its pair's first place in its group plus the pair's pixels before it there
 #pragma unroll
             for (int i = 0; i < G::kItems; ++i)
-                if (lohi[i] != 0xffffffffu)
+                if (pk[i] != 0xffffffffu)
                 {
                     const uint32_t q = pk[i], pw = pl >> 5, gw = pw / R::kGroupWords;
                     uint32_t at = r.coff[gw][q] + uint32_t(__popc(r.mask[q][pw] & ((1u << (pl & 31u)) - 1u)));
@@ -452,7 +467,7 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
                     for (int w = 0; w < R::kMaskWords; ++w)
                         if (uint32_t(w) < pw && uint32_t(w) / R::kGroupWords == gw)
                             at += __popc(r.mask[q][w]);
-                    cout[at] = uint16_t(pl | (uint32_t(vals[i]) << kPixBits));
+                    cout[at] = uint16_t(pl | (slots_of(i) << kPixBits));
                 }
             if (tid == 0)
             {
@@ -470,6 +485,10 @@ __global__ __launch_bounds__(2 * TP, 5 * 128 / TP) void k_tile_build(IndexGroup 
 
     // ---- sorting path: keys (block << 8 | pixel)
     uint32_t keys[G::kItems];
+    uint8_t vals[G::kItems];
+#pragma unroll
+    for (int i = 0; i < G::kItems; ++i)
+        vals[i] = uint8_t(slots_of(i));
 #pragma unroll
     for (int i = 0; i < G::kItems; ++i)
         keys[i] = lohi[i] == 0xffffffffu
