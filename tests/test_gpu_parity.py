@@ -476,6 +476,36 @@ def test_batch_equals_solo(torch_dev):
         say("batch member", i, "warp error vs replayed fp64", err, "flips", flips)
 
 
+@pytest.mark.parametrize("split", [False, True])
+def test_batch_sizes_equal_solo(torch_dev, split):
+    """A work-group finds its solve in the launch's map in one of three ways: of one solve, of up to 64 (one a lane),
+    and of more (a search).  Uneven small solves in batches on both sides of each limit have their solo bits."""
+    from starhub_amd import native, scene, workload
+    cfgs = [replace(scene.config_c1(seed=70 + n), num_surfels=30 * n, num_nodes=n, width=8 * w, height=6 * w,
+                    fx=7.5 * w, fy=7.5 * w, solver=replace(scene.config_c1().solver, gn_iterations=2))
+            for n, w in ((40, 9), (97, 12), (33, 7), (150, 14), (64, 11))]
+    frames = [workload.device_frame(scene.generate(c))[0] for c in cfgs]
+    flags = native.SH_FLAG_NO_PERSISTENT_PCG if split else 0
+    bcfg = native.make_config(cfgs[0].solver, 112, 84, 150, cfgs[0].K, flags=flags)
+    solo = []
+    for f in frames:
+        s = native.WarpSolver(bcfg)
+        s.process_frame(f)
+        solo.append(s.node_se3().cpu().numpy())
+        s.close()
+    assert all(np.isfinite(a).all() and not np.array_equal(a[:33], solo[2]) for a in solo[:2])
+    batch = native.BatchSolver(bcfg, 131)
+    # 131 solves have more groups than the resident PCG runs at once, and take the split one either way
+    for n in (1, 2, 63, 64, 65) + ((131,) if split else ()):
+        for i in range(n):
+            batch.set_inputs(i, frames[(i + n) % len(frames)])
+        batch.solve(n)
+        say("batch of", n, "split" if split else "")
+        for i in range(n):
+            assert np.array_equal(batch.node_se3(i).cpu().numpy(), solo[(i + n) % len(frames)]), (n, i)
+    batch.close()
+
+
 def test_pipelined_batch_subsets_equal_solo(torch_dev):
     """The pipelined PCG's tagged publications: a batch solved with 4, then
     2, then 4 members (slots idle for a launch keep stale publications) gives
