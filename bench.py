@@ -136,6 +136,7 @@ def solve_bytes(cfg, P: int, U: int) -> float:
     return index + cfg.solver.gn_iterations * per_gn
 
 
+# tiles: K = 8, as in every leg (k_tiles sums the tiles that k_tiles_matrix does not take)
 KERNEL_OF_PHASE = {"dense_terms": "k_terms", "reg_terms": "k_terms", "rows_seg": "k_rows_seg",
                    "rows_combine": "k_rows_combine", "dinv": "k_dinv", "pcg": "k_pcg_resident",
                    "update": "k_update", "tiles": "k_tiles_matrix", "tiles_combine": "k_tiles_combine"}

@@ -19,9 +19,9 @@
 // contiguous over six lanes, five lanes to a scalar row's blocks in the
 // product, and all of a lane's loads in flight before partials are summed.
 // Of more than 8192 rows a work-group takes several turns, so that the update
-// has at most 1024 partials to sum.  With one thread per 6-row block and a row's blocks one after another
-// in four kernels, 256 rows and 10 iterations took 179 us and 4096 rows and 20
-// iterations 366 us; 114 and 220 us so.
+// has at most 1024 partials to sum.  256 rows and 10 iterations take 107 us,
+// 4096 rows and 20 iterations 214 us (whole calls); with one thread per 6-row
+// block and a row's blocks one after another in four kernels 174 and 363 us.
 // Every work-group reduces the same partials in the same order, so alpha and
 // beta are the same bits everywhere; vectors are FP32 as in the reference,
 // the product's row sums, dot products, alpha and beta FP64 (cuBLAS Sdot in the reference,
@@ -48,9 +48,8 @@ constexpr int kBpGroupRows = kBpWaveRows * (kBpThreads / 64); // and of a work-g
 // 16 blocks a row, 256 / 4096 / 20000 rows: 211 / 226 / 419 us with two in
 // flight, 207 / 233 / 462 with three, 212 / 237 / 504 with four (136
 // registers, fewer waves); one lane per scalar row of the system with its
-// blocks one after another 240 / 282 us at 256 and 4096 rows; work-groups of
-// 512 and 1024 threads are slower at 256 rows (121 and 141 for 101 us at 10
-// iterations).
+// blocks one after another 240 / 282 us at 256 and 4096 rows; with work-groups
+// of 512 and 1024 threads 256 rows take a fifth and two fifths longer.
 constexpr int kBpRowBlocks = 5;
 constexpr int kBpRowLanes = 6 * kBpRowBlocks;
 constexpr int kBpAhead = 2;

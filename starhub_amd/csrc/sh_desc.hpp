@@ -78,7 +78,7 @@ struct SolveDesc
     uint8_t *gprank;         // P*K: each pixel slot's node as its rank in the tile (kNoRank: a later slot names it too)
     uint16_t *tile_group;    // n_tiles*(kTileGroups+1): first slot of each 64-pixel group of a tile, then their end
     uint16_t *slot_pair;     // S: the ranks of a slot's nodes, ra | rb << 8
-    uint16_t *tc_contrib;    // contributions, per slot in pixel order: pixel | ka << 7 | kb << 10
+    uint16_t *tc_contrib;    // contributions, per slot in pixel order: pixel | ka << 8 | kb << 11
     uint32_t *tc_slot_first; // S+1: first contribution of each slot
     uint32_t *list_off;      // N+2U+1: first entry of each block in list_items
     uint32_t *list_items;    // S: slot ids sorted by block (stable: tile order)
@@ -95,7 +95,9 @@ struct SolveDesc
     float *rhs;       // N*6  = -J^T W r
     // PCG vectors (6N each)
     float *x, *r, *s, *q, *dv[2];
-    double *mv[2];    // pipelined PCG: the exchanged vector m = M^-1 w, 6N each, by iteration parity
+    // 6N 64-bit words each, by iteration parity.  Pipelined PCG: the exchanged
+    // vector m = M^-1 w as doubles; split PCG: pairs of floats (d, s)
+    double *mv[2];
     double *delta;    // pcg_iters + 1 : r.s per iteration
     double *cost;     // weighted cost (dense + ARAP) at the start of each GN iteration, then the final one
     double *cost_part; // partials: ceil(P/64) dense (one per 64-pixel group), then ceil((E+N)/256) ARAP

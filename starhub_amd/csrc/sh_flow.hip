@@ -72,9 +72,10 @@ __device__ __forceinline__ float4 texel4(const float4 *__restrict__ m, int W, in
 // kept four times so that the lanes of a wave that name one node spread over
 // four addresses) and one global atomic per distinct node and component
 // follows.  A pixel that finds no entry within kMotionProbes adds to global
-// memory itself.  Integer sums: the same bits either way.  Bound before by
-// the serial 64-bit atomics on each node's line (1279x717, 2047 nodes: 418 us
-// before, 34 us now; 320x240, 512 nodes: 48 and 4.5 us).
+// memory itself.  Integer sums: the same bits either way.  Every pixel adding
+// to global memory is bound by the serial 64-bit atomics on a node's line
+// (1279x717, 2047 nodes: 418 us; 320x240, 512 nodes: 48 us); through the table
+// it is 34 and 4.5 us, with four LDS atomics a pixel left.
 constexpr int kMotionTile = 16;
 constexpr uint32_t kMotionSlots = 64; // entries of the table (a power of two)
 constexpr uint32_t kMotionReps = 4;

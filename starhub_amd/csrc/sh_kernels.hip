@@ -1039,11 +1039,11 @@ __device__ __forceinline__ float d_next(double beta, float dold, float s)
 // One wave takes eight block rows, a lane a scalar row, and adds its products
 // in block and column order.  Each lane reads one (d_{k-1}, s) pair of a
 // block's column, forms d_k once and hands it to the row's six lanes through
-// LDS (a lane used to gather all twelve values and form six); kU blocks are in
-// flight and the next kU on the way, without branches among the loads.  The
-// launch is bound by that chain of loads (row, column, vector): twelve solves
-// of 128 to 4096 nodes took 18.5 us with 32 rows a work-group and now take
-// 13 us.  Measured and not taken: a work-group's blocks through LDS as float4s
+// LDS, so that no lane gathers all twelve values; kU blocks are in flight and
+// the next kU on the way, without branches among the loads.  The launch is
+// bound by that chain of loads (row, column, vector): twelve solves of 128 to
+// 4096 nodes take 13.6 us (18.5 us with 32 rows a work-group, each lane
+// gathering its twelve).  Measured and not taken: a work-group's blocks through LDS as float4s
 // (16 us: its barriers and LDS cost more than its wide loads give), three
 // teams of nine lanes a row with a float4 each (12 us, but another order of
 // the sums), two or four nodes a work-group (the partials' reduction grows).
@@ -1204,7 +1204,7 @@ __global__ __launch_bounds__(kPcgThreads) void k_pcg_update(const SolveDesc *__r
     const SolveDesc d = global_desc(sds[si]);
     // everything the row needs is loaded before the partials are summed, and
     // not after: the launch is a chain of loads, and so one trip shorter
-    // (twelve solves: 5.3 to 5.0 us a launch, 60 of them a batch)
+    // (twelve solves: 5.0 us a launch, 60 of them a batch; 5.3 us otherwise)
     const float *__restrict__ dnew = pick2(d.dv, (k + 1) & 1);
     const uint32_t node = (blockIdx.x - wg_begin[si]) * kPcgNodes + threadIdx.x / 6;
     const int a = threadIdx.x % 6;

@@ -303,8 +303,8 @@ __global__ __launch_bounds__(kSkinTile) void k_skin(const float4 *__restrict__ s
 // The grid takes no memory of the caller's and none is kept between calls:
 // building it costs a work-group a few microseconds (N reads from L2), so the
 // launch is at most two 1024-thread work-groups a CU.
-// K = 8: 1.2M surfels, 4096 nodes 2335 us -> 197 us; 300k, 1024 370 -> 72 us;
-// 20k, 256 99 -> 34 us (the first: a thread per surfel scanning all nodes).
+// K = 8: 1.2M surfels, 4096 nodes 197 us; 300k, 1024 72 us; 20k, 256 34 us (a
+// thread per surfel scanning all nodes 2335, 370 and 99 us).
 // More than kGridNodes nodes take k_skin: 64 KB of nodes and 12 KB of cells
 // leave room for two work-groups a CU, and a graph of the solver has no more.
 constexpr uint32_t kGridNodes = 4096;
@@ -314,7 +314,7 @@ constexpr uint32_t kGridGroups = 512; // two for each of the 256 CUs
 constexpr uint16_t kToScan = 0xffffu; // first id of a surfel that the grid leaves to the scan (no id: N <= 4096)
 constexpr uint32_t kScanLanes = 24;   // more such surfels than this in a wave: each lane scans its own
 constexpr float kFarCells = 2.f;
-constexpr int kMaxShells = 6; // an eighth of the cells of a full grid
+constexpr int kMaxShells = 6; // at most 13^3 cells, about a third of a full grid's
 
 struct GridShape
 {
@@ -680,9 +680,12 @@ constexpr uint32_t kGraphTile = 2048;
 // UpdateNodeDistanceKernel + BuildNodeGraphKernel + BuildNodeGraphPairKernel
 // + ResetNodeConnectionKernel (NodeGraph.cu:10-145): the FP16 distance of each
 // pair is recomputed on the fly instead of being stored as an N x N matrix.
-// One wave per node: a thread per node (one work-group per 256 nodes) left
-// most CUs without work and scanned its N candidates one after another
-// (K = 8: 4096 nodes 818 us -> 35 us, 256 nodes 112 -> 15 us).
+// The compiler makes a distance's last multiply-add and its conversion one
+// instruction, which rounds once, straight to 16 bits: where the 32-bit value
+// would lie midway between two 16-bit ones, the result may be the other one.
+// One wave per node, so that few nodes fill the chip too and a step looks at
+// 64 candidates; bound by the step's chain of ballots and list updates (K = 8:
+// 4096 nodes 35 us, 256 nodes 15 us; with a thread per node 818 and 112 us).
 template <int K>
 __global__ __launch_bounds__(kGraphThreads) void k_node_graph(const float4 *__restrict__ nodes, uint32_t N, float r2,
                                                               uint16_t *__restrict__ node_knn,

@@ -209,13 +209,13 @@ __device__ float3 smallest_eigvec(const float cov[6])
 }
 
 // A window point as the tiles hold it: w = 1, or all zeros where there is no
-// valid vertex (zero_vertex), tested once per texel instead of once per window
-// that holds it (85 times).  A zero adds nothing to the window sums, and
-// the covariance takes its difference as 0, so neither loop branches.
-// With the window's rows not unrolled and no array indexed at run time the
-// kernels hold 52 registers instead of 190 and keep eight waves a SIMD, not
-// two; they are bound by the window's arithmetic (1279x717: filter 64 -> 33 us,
-// normals 61 -> 31 us).
+// valid vertex (zero_vertex), so that a texel is tested once and not by each
+// of the windows that hold it (85 points a window).  A zero adds nothing to
+// the window sums, and the covariance takes its difference as 0, so neither
+// loop branches.  The sums are FP32, 85 16-byte LDS reads a window; with the
+// window's rows not unrolled and no array indexed at run time the kernels hold
+// 52 registers and keep eight waves a SIMD (1279x717: filter 33 us, normals 31
+// us; 190 registers, two waves and a test per point 64 and 61 us).
 __device__ __forceinline__ float4 window_point(float x, float y, float z)
 {
     return zero_vertex(x, y, z) ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(x, y, z, 1.f);
