@@ -12,14 +12,15 @@
 //   k_bp_update  alpha = delta / (d.q); x += alpha d; t = r - alpha q;
 //                s = M^-1 t; partial sums of t.s
 // With an operator of the caller's (a host callback that enqueues on the
-// solve's stream) the product needs d in memory, and it is four, to the same
-// bits: the callback, k_bp_dot (partials of d.q), k_bp_update, k_bp_dir (d).
+// solve's stream) the product needs d in memory, and it is four: the callback,
+// k_bp_dot (partials of d.q), k_bp_update, k_bp_dir (d).  To the same bits up
+// to 8192 rows; of more, where the two forms of the product differ, the
+// partials of d.q may be of other rows.
 // Bound by launches and by the latency of each kernel's dependent loads, not
 // by bandwidth: one lane per scalar row of a block, so that loads are
 // contiguous over six lanes, five lanes to a scalar row's blocks in the
 // product, and all of a lane's loads in flight before partials are summed.
-// Of more than 8192 rows a work-group takes several turns, so that the update
-// has at most 1024 partials to sum.  256 rows and 10 iterations take 107 us,
+// Work-groups take turns so that there are at most 1024 partials.  256 rows and 10 iterations take 107 us,
 // 4096 rows and 20 iterations 214 us (whole calls); with one thread per 6-row
 // block and a row's blocks one after another in four kernels 174 and 363 us.
 // Every work-group reduces the same partials in the same order, so alpha and
@@ -56,6 +57,26 @@ constexpr int kBpAhead = 2;
 constexpr int kBpSpmvThreads = 256;
 constexpr int kBpSpmvRows = 2 * (kBpSpmvThreads / 64); // rows of a work-group in one turn
 constexpr uint32_t kBpSpmvGroups = 1024;           // more rows than these take turns
+// Larger systems: at kBpSharedRows the work-group begins to sum the partials
+// together (each wave for itself, a wave's loads are too many), and the row
+// kernels take turns past kBpRowGroups (1024 and not 2048: 60000 rows 303 and
+// 316 us).  With at most kBpLongBlocks blocks a row the product takes one lane
+// per scalar row there, as the row kernels do: the rows fill the chip by
+// themselves, and five lanes to one would mostly idle.  From kBpApartBlocks on
+// the product is a kernel of its own for the built-in operator too: it gathers
+// d alone then, not s and d, and is long against a launch.  Ten iterations, us:
+//   rows x blocks   pairs of rows  lane a row  apart
+//   10000 x 11      146            134         155
+//   16384 x 25      222            260         231
+//   32768 x 11      265            222         251
+//   60000 x 5       293            196         217
+//   60000 x 11      309            299         312
+//   60000 x 25      546            586         486
+//   150000 x 11     1027           782         660
+constexpr uint32_t kBpSharedRows = kBpSpmvRows * kBpSpmvGroups + 1;
+constexpr uint32_t kBpRowGroups = 1024;
+constexpr uint32_t kBpLongBlocks = 16;
+constexpr uint32_t kBpApartBlocks = 1u << 20;
 
 // A lane's scalar row: row 6 * row + a of the system, in the wave's lane 6 * (row of the wave) + a
 struct BpLane
@@ -65,41 +86,71 @@ struct BpLane
     bool on;
 };
 
-__device__ inline BpLane bp_lane(uint32_t nblk)
+__device__ inline BpLane bp_lane(uint32_t row0, uint32_t nblk)
 {
     const uint32_t lane = threadIdx.x % 64u, wave = threadIdx.x / 64u;
     BpLane l;
     l.a = lane % 6u;
     l.first = int(lane - l.a);
-    const uint32_t row = blockIdx.x * kBpGroupRows + wave * kBpWaveRows + lane / 6u;
+    const uint32_t row = row0 + wave * kBpWaveRows + lane / 6u;
     l.on = lane < 6u * kBpWaveRows && row < nblk;
     l.row = min(row, nblk - 1u);
     l.i = 6u * l.row + l.a;
     return l;
 }
 
-// Sum of `n` FP64 partials in a fixed order (lane j takes j, j+64, ...; then a
-// fixed shuffle tree); every wave that calls it gets the same bits.  Eight
+// f(row0) for each turn of a row kernel's work-group: one where there are no turns
+template <bool TURNS, class F>
+__device__ inline void bp_turns(uint32_t nblk, F f)
+{
+    if constexpr (TURNS)
+        for (uint32_t row0 = blockIdx.x * kBpGroupRows; row0 < nblk; row0 += gridDim.x * kBpGroupRows)
+            f(row0);
+    else
+        f(blockIdx.x * kBpGroupRows);
+}
+
+// This lane's part of the sum of `n` FP64 partials: lane j of a wave takes j,
+// j + 64, ...; SHARED: thread j of the work-group takes j, j + 256, ....  Eight
 // loads in flight, past the end the last partial again.
+template <bool SHARED>
 __device__ inline double lane_partials(const double *__restrict__ part, uint32_t n)
 {
+    constexpr uint32_t kStep = SHARED ? kBpThreads : 64u;
     double v = 0.0;
-    for (uint32_t i = threadIdx.x % 64u; i < n; i += 8 * 64)
+    for (uint32_t i = threadIdx.x % kStep; i < n; i += 8 * kStep)
     {
         double p[8];
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u)
-            p[u] = part[min(i + 64u * u, n - 1u)];
+            p[u] = part[min(i + kStep * u, n - 1u)];
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u)
-            v = i + 64u * u < n ? v + p[u] : v;
+            v = i + kStep * u < n ? v + p[u] : v;
     }
     return v;
 }
 
-__device__ inline double sum_partials(const double *__restrict__ part, uint32_t n)
+// The partials' sum from the lanes' parts, in a fixed order: a shuffle tree,
+// by every wave for itself, or (SHARED) over the work-group, whose waves' sums
+// are added in wave order; the same bits in every wave.  SHARED: all threads
+// call it, once a kernel.
+template <bool SHARED>
+__device__ inline double sum_partials(double lane_sum)
 {
-    return wave_sum(lane_partials(part, n));
+    double v = wave_sum(lane_sum);
+    if constexpr (SHARED)
+    {
+        __shared__ double ws[kBpThreads / 64];
+        if (threadIdx.x % 64u == 0)
+            ws[threadIdx.x / 64u] = v;
+        __syncthreads();
+        v = ws[0];
+#pragma unroll
+        for (int w = 1; w < kBpThreads / 64; ++w)
+            v += ws[w];
+    }
+    return v;
 }
 
 // Work-group sum of one value per thread, in a fixed order: wave sums, then
@@ -148,29 +199,35 @@ __device__ inline float precond6(const BpInvRow &mi, float v, const BpLane &l)
 
 // r = b, x = 0 (zero_init) or r given (InitResidual already ran); s = M^-1 r;
 // partials of r.s  (blockPCGZeroInitKernel / Initialize, BlockPCG.cuh:395-440)
+template <bool SHARED>
 __global__ void k_bp_init(const float *__restrict__ b, const float *__restrict__ minv, float *__restrict__ r,
                           float *__restrict__ s, float *__restrict__ x, uint32_t nblk, int zero_init,
                           double *__restrict__ part)
 {
-    const BpLane l = bp_lane(nblk);
-    const float rv = zero_init ? b[l.i] : r[l.i];
-    const float y = precond6(load_inv(minv, l), rv, l);
-    if (l.on)
-    {
-        if (zero_init)
+    double rs = 0.0;
+    bp_turns<SHARED>(nblk, [&](uint32_t row0) __attribute__((always_inline)) {
+        const BpLane l = bp_lane(row0, nblk);
+        const float rv = zero_init ? b[l.i] : r[l.i];
+        const float y = precond6(load_inv(minv, l), rv, l);
+        if (l.on)
         {
-            r[l.i] = rv;
-            x[l.i] = 0.f;
+            if (zero_init)
+            {
+                r[l.i] = rv;
+                x[l.i] = 0.f;
+            }
+            s[l.i] = y;
         }
-        s[l.i] = y;
-    }
-    block_sum_store(l.on ? double(y) * double(rv) : 0.0, part + blockIdx.x);
+        rs += l.on ? double(y) * double(rv) : 0.0;
+    });
+    block_sum_store(rs, part + blockIdx.x);
 }
 
-// delta[it] = sum of the partials (one wave)
+// delta[it] = sum of the partials (one wave; SHARED: one work-group)
+template <bool SHARED>
 __global__ void k_bp_delta(const double *__restrict__ part, uint32_t n, double *__restrict__ delta, uint32_t it)
 {
-    const double s = sum_partials(part, n);
+    const double s = sum_partials<SHARED>(lane_partials<SHARED>(part, n));
     if (threadIdx.x == 0)
         delta[it] = s;
 }
@@ -204,64 +261,95 @@ __device__ inline BpRowLane bp_row_lane()
 }
 
 // the dot product d.q over the lanes and turns of k_bp_spmv
+template <bool LONG>
 __global__ void k_bp_dot(const float *__restrict__ d, const float *__restrict__ q, uint32_t nblk,
                          double *__restrict__ part)
 {
-    const BpRowLane l = bp_row_lane();
+    constexpr uint32_t kRows = LONG ? kBpGroupRows : kBpSpmvRows;
     double v = 0.0;
-    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nblk; row0 += gridDim.x * kBpSpmvRows)
+    for (uint32_t row0 = blockIdx.x * kRows; row0 < nblk; row0 += gridDim.x * kRows)
     {
-        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
-        if (l.lead && row < nblk)
-            v += double(d[6 * size_t(row) + l.a]) * double(q[6 * size_t(row) + l.a]);
+        if constexpr (LONG)
+        {
+            const BpLane l = bp_lane(row0, nblk);
+            if (l.on)
+                v += double(d[l.i]) * double(q[l.i]);
+        }
+        else
+        {
+            const BpRowLane l = bp_row_lane();
+            const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+            if (l.lead && row < nblk)
+                v += double(d[6 * size_t(row) + l.a]) * double(q[6 * size_t(row) + l.a]);
+        }
     }
     block_sum_store<kBpSpmvThreads>(v, part + blockIdx.x);
 }
 
 // the second kernel of the reference's iteration (BlockPCG.cuh:442-472)
+template <bool SHARED>
 __global__ void k_bp_update(float *__restrict__ x, const float *__restrict__ r, const float *__restrict__ d,
                             const float *__restrict__ q, const float *__restrict__ minv, float *__restrict__ t,
                             float *__restrict__ s, uint32_t nblk, const double *__restrict__ part_dq,
                             uint32_t n_dq, const double *__restrict__ delta, uint32_t it,
                             double *__restrict__ part_ts)
 {
-    const BpLane l = bp_lane(nblk);
-    // everything is loaded before the partials are summed
-    const double delta_it = delta[it];
-    const float xv = x[l.i], rv = r[l.i], dv = d[l.i], qv = q[l.i];
-    const BpInvRow mi = load_inv(minv, l);
-    const double dq = sum_partials(part_dq, n_dq);
-    const float a = float(dq != 0.0 ? delta_it / dq : 0.0);
-    const float tv = rv - a * qv;
-    const float y = precond6(mi, tv, l);
-    if (l.on)
-    {
-        x[l.i] = xv + a * dv;
-        t[l.i] = tv;
-        s[l.i] = y;
-    }
-    block_sum_store(l.on ? double(y) * double(tv) : 0.0, part_ts + blockIdx.x);
+    double ts = 0.0;
+    float a = 0.f;
+    bool first = true;
+    bp_turns<SHARED>(nblk, [&](uint32_t row0) __attribute__((always_inline)) {
+        const BpLane l = bp_lane(row0, nblk);
+        // everything is loaded before the partials are summed
+        const double delta_it = delta[it];
+        const float xv = x[l.i], rv = r[l.i], dv = d[l.i], qv = q[l.i];
+        const BpInvRow mi = load_inv(minv, l);
+        if (first)
+        {
+            const double dq = sum_partials<SHARED>(lane_partials<SHARED>(part_dq, n_dq));
+            a = float(dq != 0.0 ? delta_it / dq : 0.0);
+            first = false;
+        }
+        const float tv = rv - a * qv;
+        const float y = precond6(mi, tv, l);
+        if (l.on)
+        {
+            x[l.i] = xv + a * dv;
+            t[l.i] = tv;
+            s[l.i] = y;
+        }
+        ts += l.on ? double(y) * double(tv) : 0.0;
+    });
+    block_sum_store(ts, part_ts + blockIdx.x);
 }
 
-// delta' = t.s and beta = delta' / delta of iteration it, by a whole wave from
-// its lanes' sums; the first work-group keeps delta' for the update and the history
+// delta' = t.s and beta = delta' / delta of iteration it, from the lanes' sums;
+// the first work-group keeps delta' for the update and the history
+template <bool SHARED>
 __device__ inline float bp_beta(double lane_sum, double *__restrict__ delta, uint32_t it)
 {
     const double dold = it ? delta[it - 1] : 0.0;
-    const double dn = wave_sum(lane_sum);
+    const double dn = sum_partials<SHARED>(lane_sum);
     if (blockIdx.x == 0 && threadIdx.x == 0)
         delta[it] = dn;
     return float(dold != 0.0 ? dn / dold : 0.0);
 }
 
 // the third kernel (BlockPCG.cuh:474-483): d = s + beta d; delta[it] = t.s (iteration 0: d = s)
+template <bool SHARED>
 __global__ void k_bp_dir(const float *__restrict__ s, float *__restrict__ d, uint32_t nblk,
-                         const double *__restrict__ part_ts, double *__restrict__ delta, uint32_t it)
+                         const double *__restrict__ part_ts, uint32_t n_ts, double *__restrict__ delta, uint32_t it)
 {
-    const BpLane l = bp_lane(nblk);
-    const float beta = bp_beta(lane_partials(part_ts, gridDim.x), delta, it);
-    if (l.on)
-        d[l.i] = it ? s[l.i] + beta * d[l.i] : s[l.i];
+    float beta = 0.f;
+    bool first = true;
+    bp_turns<SHARED>(nblk, [&](uint32_t row0) __attribute__((always_inline)) {
+        const BpLane l = bp_lane(row0, nblk);
+        const float sv = s[l.i], dv = it ? d[l.i] : 0.f;
+        if (first)
+            beta = bp_beta<SHARED>(lane_partials<SHARED>(part_ts, n_ts), delta, it);
+        first = false;
+        if (l.on)
+            d[l.i] = it ? sv + beta * dv : sv;
+    });
 }
 
 struct BpVector // a vector in memory
@@ -362,18 +450,56 @@ __device__ inline float bcsr_row(const uint32_t *__restrict__ row_ptr, const uin
     return float(pair + __shfl(pair, lane + 6, 64) + fifth);
 }
 
+// The same by one lane, a block after another: for long systems, whose rows
+// fill the chip by themselves.  Bound by the blocks' bytes; unrolled, four
+// blocks' loads at a time (150000 rows of 11 blocks 43 us, a pair of rows a
+// wave 48, one block ahead without the unrolling 46).  The row of m is copied
+// before the vector is asked for: otherwise the loads stay one by one (the
+// fused product at 32768 rows 279 and not 222 us in ten iterations).
+template <class V, class F>
+__device__ inline float bcsr_long_row(const uint32_t *__restrict__ row_ptr, const uint32_t *__restrict__ col,
+                                      const float *__restrict__ blocks, const BpLane &l, V &v, F ready)
+{
+    const uint32_t k0 = row_ptr[l.row], k1 = row_ptr[l.row + 1];
+    ready();
+    double acc = 0.0;
+#pragma unroll 4
+    for (uint32_t k = k0; k < k1; ++k)
+    {
+        const float *blk = blocks + 36 * size_t(k) + 6 * l.a;
+        float m[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+            m[c] = blk[c];
+        typename V::Entries e;
+        v.load(col[k], e);
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+            acc = fma(double(m[c]), double(v.value(e, c)), acc);
+    }
+    return float(acc);
+}
+
 // y = A x, or y = b - A x (b: InitResidual's r = b - A x)
+template <bool LONG>
 __global__ __launch_bounds__(kBpSpmvThreads) void k_bcsr_spmv(const uint32_t *__restrict__ row_ptr,
                                                           const uint32_t *__restrict__ col,
                                                           const float *__restrict__ blocks, const float *__restrict__ x,
                                                           const float *__restrict__ b, float *__restrict__ y,
                                                           uint32_t nrows)
 {
-    const BpRowLane l = bp_row_lane();
     const BpVector v{x};
-    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nrows; row0 += gridDim.x * kBpSpmvRows)
+    if constexpr (LONG)
     {
-        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+        const BpLane l = bp_lane(blockIdx.x * kBpGroupRows, nrows);
+        const float acc = bcsr_long_row(row_ptr, col, blocks, l, v, [] {});
+        if (l.on)
+            y[l.i] = b ? b[l.i] - acc : acc;
+    }
+    else
+    {
+        const BpRowLane l = bp_row_lane();
+        const uint32_t row = blockIdx.x * kBpSpmvRows + (threadIdx.x / 64u) * 2u + l.r;
         const size_t i = 6 * size_t(row) + l.a;
         const float acc = bcsr_row(row_ptr, col, blocks, min(row, nrows - 1u), l, v, [] {});
         if (l.lead && row < nrows)
@@ -384,6 +510,7 @@ __global__ __launch_bounds__(kBpSpmvThreads) void k_bcsr_spmv(const uint32_t *__
 // k_bp_dir, k_bcsr_spmv and k_bp_dot in one: the direction is formed where it
 // is gathered, from s and the old direction, and each row stores its own part
 // of the new one (another buffer: other rows still read the old)
+template <bool SHARED, bool LONG>
 __global__ __launch_bounds__(kBpSpmvThreads) void k_bp_spmv(const uint32_t *__restrict__ row_ptr,
                                                         const uint32_t *__restrict__ col,
                                                         const float *__restrict__ blocks, const float *__restrict__ s,
@@ -393,22 +520,39 @@ __global__ __launch_bounds__(kBpSpmvThreads) void k_bp_spmv(const uint32_t *__re
                                                         double *__restrict__ delta, uint32_t it,
                                                         double *__restrict__ part_dq)
 {
-    const BpRowLane l = bp_row_lane();
-    const double ts = lane_partials(part_ts, n_ts);
+    const double ts = lane_partials<SHARED>(part_ts, n_ts);
     BpDirection v{s, it ? d_old : s, it != 0u, 0.f};
     bool first = true;
+    auto ready = [&] {
+        if (first)
+            v.beta = bp_beta<SHARED>(ts, delta, it);
+        first = false;
+    };
     double dq = 0.0;
-    for (uint32_t row0 = blockIdx.x * kBpSpmvRows; row0 < nblk; row0 += gridDim.x * kBpSpmvRows)
+    constexpr uint32_t kRows = LONG ? kBpGroupRows : kBpSpmvRows;
+    for (uint32_t row0 = blockIdx.x * kRows; row0 < nblk; row0 += gridDim.x * kRows)
     {
-        const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
-        const size_t i = 6 * size_t(min(row, nblk - 1u)) + l.a;
-        const float sv = s[i], ov = v.d[i];
-        const float acc = bcsr_row(row_ptr, col, blocks, min(row, nblk - 1u), l, v, [&] {
-            if (first)
-                v.beta = bp_beta(ts, delta, it);
-            first = false;
-        });
-        if (l.lead && row < nblk)
+        bool own;
+        size_t i;
+        float sv, ov, acc;
+        if constexpr (LONG)
+        {
+            const BpLane l = bp_lane(row0, nblk);
+            own = l.on;
+            i = l.i;
+            sv = s[i], ov = v.d[i];
+            acc = bcsr_long_row(row_ptr, col, blocks, l, v, ready);
+        }
+        else
+        {
+            const BpRowLane l = bp_row_lane();
+            const uint32_t row = row0 + (threadIdx.x / 64u) * 2u + l.r;
+            own = l.lead && row < nblk;
+            i = 6 * size_t(min(row, nblk - 1u)) + l.a;
+            sv = s[i], ov = v.d[i];
+            acc = bcsr_row(row_ptr, col, blocks, min(row, nblk - 1u), l, v, ready);
+        }
+        if (own)
         {
             const float dv = it ? sv + v.beta * ov : sv;
             d[i] = dv;
@@ -437,11 +581,25 @@ __global__ void k_bcsr_check(const uint32_t *__restrict__ row_ptr, const uint32_
 }
 
 inline uint32_t grid_of(uint32_t n) { return (n + kBpThreads - 1) / kBpThreads; }
-inline uint32_t spmv_grid(uint32_t nblk)
+inline uint32_t row_groups(uint32_t nblk) { return (nblk + kBpGroupRows - 1) / kBpGroupRows; }
+inline uint32_t row_grid(uint32_t nblk) { return std::min(row_groups(nblk), kBpRowGroups); }
+inline uint32_t pair_groups(uint32_t nblk) { return (nblk + kBpSpmvRows - 1) / kBpSpmvRows; } // two rows a wave
+inline uint32_t pair_grid(uint32_t nblk) { return std::min(pair_groups(nblk), kBpSpmvGroups); }
+inline bool long_rows(uint32_t nblk, uint32_t nnz)
 {
-    return std::min((nblk + kBpSpmvRows - 1) / kBpSpmvRows, kBpSpmvGroups);
+    return nblk >= kBpSharedRows && nnz / kBpLongBlocks <= nblk;
 }
-inline uint32_t row_grid(uint32_t nblk) { return (nblk + kBpGroupRows - 1) / kBpGroupRows; }
+
+// y = A x or b - A x
+void start_bcsr_spmv(const uint32_t *row_ptr, const uint32_t *col, const float *blocks, const float *x, const float *b,
+                     float *y, uint32_t rows, uint32_t nnz, hipStream_t st)
+{
+    if (long_rows(rows, nnz))
+        hipLaunchKernelGGL(k_bcsr_spmv<true>, dim3(row_groups(rows)), dim3(kBpSpmvThreads), 0, st, row_ptr, col, blocks,
+                           x, b, y, rows);
+    else
+        hipLaunchKernelGGL(k_bcsr_spmv<false>, dim3(pair_groups(rows)), dim3(kBpSpmvThreads), 0, st, row_ptr, col, blocks, x, b, y, rows);
+}
 
 int status_of(hipError_t e)
 {
@@ -559,9 +717,8 @@ extern "C"
     {
         if (!spmv || !x || !y)
             return SH_E_ARG;
-        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::spmv_grid(spmv->rows)), dim3(sh::kBpSpmvThreads), 0,
-                           reinterpret_cast<hipStream_t>(stream), spmv->row_ptr, spmv->col, spmv->blocks, x,
-                           static_cast<const float *>(nullptr), y, spmv->rows);
+        sh::start_bcsr_spmv(spmv->row_ptr, spmv->col, spmv->blocks, x, nullptr, y, spmv->rows, spmv->nnz,
+                            reinterpret_cast<hipStream_t>(stream));
         return sh::status_of(hipGetLastError());
     }
 
@@ -570,9 +727,8 @@ extern "C"
     {
         if (!spmv || !x_init || !b || !residual)
             return SH_E_ARG;
-        hipLaunchKernelGGL(sh::k_bcsr_spmv, dim3(sh::spmv_grid(spmv->rows)), dim3(sh::kBpSpmvThreads), 0,
-                           reinterpret_cast<hipStream_t>(stream), spmv->row_ptr, spmv->col, spmv->blocks, x_init, b,
-                           residual, spmv->rows);
+        sh::start_bcsr_spmv(spmv->row_ptr, spmv->col, spmv->blocks, x_init, b, residual, spmv->rows, spmv->nnz,
+                            reinterpret_cast<hipStream_t>(stream));
         return sh::status_of(hipGetLastError());
     }
 
@@ -604,7 +760,7 @@ extern "C"
         sh_block_pcg *p = new sh_block_pcg();
         p->cap = max_matrix_size;
         const size_t vb = (size_t(max_matrix_size) * 4 + 255) / 256 * 256; // a vector's stride
-        const size_t na = sh::spmv_grid(max_matrix_size / 6u), nb = sh::row_grid(max_matrix_size / 6u);
+        const size_t na = std::max(sh::pair_grid(max_matrix_size / 6u), sh::row_grid(max_matrix_size / 6u)), nb = sh::row_grid(max_matrix_size / 6u);
         const bool ok = hipMalloc(&p->block, 6 * vb + (na + nb) * 8) == hipSuccess && ensure_delta(p, 16) == SH_OK;
         float **const vec[6] = {&p->r, &p->t, &p->d, &p->d_old, &p->q, &p->s};
         for (int i = 0; ok && i < 6; ++i)
@@ -660,7 +816,7 @@ extern "C"
         if (rc != SH_OK)
             return rc;
         const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-        const uint32_t nblk = pcg->n / 6u, g = sh::row_grid(nblk), gq = sh::spmv_grid(nblk);
+        const uint32_t nblk = pcg->n / 6u, g = sh::row_grid(nblk);
         pcg->last_iters = 0;
         if (!zero_init)
         {
@@ -677,11 +833,13 @@ extern "C"
                 return rc;
         }
         // s = M^-1 r and the partials of r.s; each iteration begins with their sum
-        hipLaunchKernelGGL(sh::k_bp_init, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->b, pcg->inv_diag, pcg->r,
-                           pcg->s, pcg->x, nblk, zero_init ? 1 : 0, pcg->part_b);
+        const bool shared = nblk >= sh::kBpSharedRows;
+        hipLaunchKernelGGL(shared ? sh::k_bp_init<true> : sh::k_bp_init<false>, dim3(g), dim3(sh::kBpThreads), 0, st,
+                           pcg->b, pcg->inv_diag, pcg->r, pcg->s, pcg->x, nblk, zero_init ? 1 : 0, pcg->part_b);
         // the sum by itself, where the host or the history needs it and no iteration follows
         auto store_delta = [&](uint32_t it) {
-            hipLaunchKernelGGL(sh::k_bp_delta, dim3(1), dim3(64), 0, st, pcg->part_b, g, pcg->delta, it);
+            hipLaunchKernelGGL(shared ? sh::k_bp_delta<true> : sh::k_bp_delta<false>, dim3(1),
+                               dim3(shared ? sh::kBpThreads : 64), 0, st, pcg->part_b, g, pcg->delta, it);
         };
         if (epsilon > 0.f || max_iterations == 0)
             store_delta(0);
@@ -694,28 +852,40 @@ extern "C"
         // the built-in product takes the direction and the dot product into its
         // kernel; any other operator needs the direction in memory
         const sh_spmv *own = pcg->ops.apply_spmv == bcsr_apply_cb ? static_cast<const sh_spmv *>(pcg->ops.user) : nullptr;
-        if (own && own->rows != nblk)
+        if (own && (own->rows != nblk || own->nnz >= sh::kBpApartBlocks))
             own = nullptr;
+        const bool by_lane = own ? sh::long_rows(nblk, own->nnz) : shared; // the lanes that hold d.q's terms
+        const uint32_t gq = by_lane ? g : sh::pair_grid(nblk);
         float *r = pcg->r, *t = pcg->t, *d = pcg->d, *d_old = pcg->d_old;
         for (uint32_t it = 0; it < max_iterations; ++it)
         {
             if (own)
             {
-                hipLaunchKernelGGL(sh::k_bp_spmv, dim3(gq), dim3(sh::kBpSpmvThreads), 0, st, own->row_ptr, own->col,
-                                   own->blocks, pcg->s, d_old, d, pcg->q, nblk, pcg->part_b, g, pcg->delta, it,
-                                   pcg->part_a);
+                auto spmv = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3(gq), dim3(sh::kBpSpmvThreads), 0, st, own->row_ptr, own->col,
+                                       own->blocks, pcg->s, d_old, d, pcg->q, nblk, pcg->part_b, g, pcg->delta, it,
+                                       pcg->part_a);
+                };
+                if (by_lane)
+                    spmv(sh::k_bp_spmv<true, true>);
+                else if (shared)
+                    spmv(sh::k_bp_spmv<true, false>);
+                else
+                    spmv(sh::k_bp_spmv<false, false>);
             }
             else
             {
-                hipLaunchKernelGGL(sh::k_bp_dir, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->s, d, nblk, pcg->part_b,
-                                   pcg->delta, it);
+                hipLaunchKernelGGL(shared ? sh::k_bp_dir<true> : sh::k_bp_dir<false>, dim3(g), dim3(sh::kBpThreads), 0,
+                                   st, pcg->s, d, nblk, pcg->part_b, g, pcg->delta, it);
                 if ((rc = sh::status_of(hipGetLastError())) != SH_OK ||
                     (rc = pcg->ops.apply_spmv(pcg->ops.user, d, pcg->q, stream)) != SH_OK)
                     return rc;
-                hipLaunchKernelGGL(sh::k_bp_dot, dim3(gq), dim3(sh::kBpSpmvThreads), 0, st, d, pcg->q, nblk, pcg->part_a);
+                hipLaunchKernelGGL(by_lane ? sh::k_bp_dot<true> : sh::k_bp_dot<false>, dim3(gq),
+                                   dim3(sh::kBpSpmvThreads), 0, st, d, pcg->q, nblk, pcg->part_a);
             }
-            hipLaunchKernelGGL(sh::k_bp_update, dim3(g), dim3(sh::kBpThreads), 0, st, pcg->x, r, d, pcg->q,
-                               pcg->inv_diag, t, pcg->s, nblk, pcg->part_a, gq, pcg->delta, it, pcg->part_b);
+            hipLaunchKernelGGL(shared ? sh::k_bp_update<true> : sh::k_bp_update<false>, dim3(g), dim3(sh::kBpThreads), 0,
+                               st, pcg->x, r, d, pcg->q, pcg->inv_diag, t, pcg->s, nblk, pcg->part_a, gq, pcg->delta,
+                               it, pcg->part_b);
             if (epsilon > 0.f || it + 1 == max_iterations)
                 store_delta(it + 1);
             if ((rc = sh::status_of(hipGetLastError())) != SH_OK)

@@ -226,3 +226,58 @@ def test_block_csr_sizes(rows, degree):
         pcg.close()
     assert np.isfinite(outs[0][0]).all() and outs[0][1].shape == (5,)
     assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("rows,degree", [(8192, 40), (8193, 15), (8193, 17), (9001, 40), (41003, 6), (45001, 25)])
+def test_block_csr_long_systems(rows, degree):
+    """Both sides of 8192 rows and of 16 blocks a row, more rows than the row kernels' work-groups take in a turn, and
+    enough blocks that the built-in product is a kernel of its own: the product is the exact sum rounded once, and the
+    built-in operator's iterations are the callback's (where their sums of d.q group rows alike, bit for bit)."""
+    import torch
+    from starhub_amd import native
+    torch.cuda.set_device(0)
+    rng = np.random.default_rng(rows + degree)
+    step = np.sort(rng.choice(np.arange(1, 3 * degree + 9), degree - 1, replace=False))
+    col = np.sort((np.arange(rows)[:, None] + np.concatenate([[0], step])[None]) % rows, 1)
+    own = torch.from_numpy(col == np.arange(rows)[:, None]).cuda()
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    blk = torch.randn(rows, degree, 6, 6, generator=g, device="cuda") * 0.02
+    blk[own] = 0.5 * (blk[own] + blk[own].transpose(1, 2)) + 3 * torch.eye(6, device="cuda")
+    dinv = torch.linalg.inv(blk[own].double().cpu()).float().cuda().contiguous()
+    b = torch.randn(6 * rows, generator=g, device="cuda")
+    A = native.BlockCsr(_dev(torch, np.arange(rows + 1, dtype=np.uint32) * degree), _dev(torch, col.astype(np.uint32).reshape(-1)),
+                        blk.reshape(-1))
+    assert A.check() == 0
+    y = torch.full_like(b, float("nan"))
+    assert A.apply(b.data_ptr(), y.data_ptr()) == 0
+    prod = blk.double() * b.double().view(-1, 6)[torch.from_numpy(col).cuda()][:, :, None, :]
+    exact, size = prod.sum((1, 3)).reshape(-1), prod.abs().sum((1, 3)).reshape(-1)
+    torch.cuda.synchronize()
+    err = (y.double() - exact).abs()
+    print("rows", rows, "degree", degree, "max err", err.max().item(), flush=True)
+    assert bool((err <= 2.0 ** -24 * exact.abs() + 2.0 ** -44 * size).all())
+
+    @native.SPMV_APPLY_FN
+    def apply(user, xp, yp, stream):
+        return A.apply(xp, yp)
+
+    outs = []
+    for ops in (A.ops(), native.SpmvOps(None, 6 * rows, apply, native.SPMV_INIT_FN())):
+        pcg = native.BlockPCG(6 * rows)
+        x = torch.full((6 * rows,), 0.25, device="cuda")
+        assert pcg.set_input(dinv, ops, b, x) == 0
+        pcg.solve(4, zero_init=False)
+        outs.append((x.cpu().numpy(), pcg.delta_history()))
+        n = pcg.solve_converge_checked(40, True, 1e-3)
+        outs[-1] += (x.cpu().numpy(), n)
+        pcg.close()
+    assert np.isfinite(outs[0][0]).all() and outs[0][1].shape == (5,) and 0 < outs[0][3] < 40
+    if rows <= 8192 or degree <= 16 or rows * degree >= 1 << 20:
+        assert all(np.array_equal(u, v) for u, v in zip(*outs))
+    else:  # sums of d.q in another order: 2^-53 of them, a rounding of 2^-24 in a few entries of a vector
+        assert all(np.allclose(u, v, rtol=1e-5, atol=1e-6) for u, v in zip(*outs))
+    # the residual the converge-checked solve stopped at
+    assert A.apply(x.data_ptr(), y.data_ptr()) == 0
+    r = (b - y).view(-1, 6, 1)
+    torch.cuda.synchronize()
+    assert float((r * (dinv.view(-1, 6, 6) @ r)).sum()) <= 1.01e-6 * float((b.view(-1, 6, 1) * (dinv.view(-1, 6, 6) @ b.view(-1, 6, 1))).sum())
