@@ -11,7 +11,8 @@
 //   k_skin_grid   finds each surfel's K nearest through a uniform grid over
 //                 the nodes, and rescans the nodes in index order for the
 //                 surfels that meet an equal distance among them;
-//   k_skin        the scan alone, for more nodes than the grid's LDS holds;
+//   k_skin        the scan alone, for few nodes and for more than the grid's
+//                 LDS holds;
 //   k_node_graph  the scan (16-bit distances are equal often), one wave per
 //                 node, 64 candidates a step.
 #include "sh_common.hpp"
@@ -185,16 +186,17 @@ struct WaveScan
         m = dpp_max<0x141>(m);         // the other four of the eight (row_half_mirror)
         max_d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), 0));
     }
-    __device__ __forceinline__ void init(float d0)
+    uint32_t lane;
+    __device__ __forceinline__ void init(float d0, uint32_t ln)
     {
-        dist = (threadIdx.x & 63u) < uint32_t(K) ? d0 : -1.f;
+        lane = ln;
+        dist = lane < uint32_t(K) ? d0 : -1.f;
         idx = 0;
         max_d = d0;
     }
     // d: this lane's candidate, node base + lane (not below any entry where there is none)
     __device__ __forceinline__ void step(uint32_t base, float d)
     {
-        const uint32_t lane = threadIdx.x & 63u;
         unsigned long long m = __ballot(d < max_d);
         while (m)
         {
@@ -259,6 +261,39 @@ __device__ __forceinline__ void store_scanned(const float4 *__restrict__ nodes, 
     }
 }
 
+// Surfel s at v (the same in all lanes) scanned by the wave over the nodes in LDS
+template <int K>
+__device__ __forceinline__ void scan_by_wave(const float4 *__restrict__ nodes, uint32_t N, float4 v, float r2, uint32_t s,
+                                             uint16_t *__restrict__ knn, float *__restrict__ spatial,
+                                             float *__restrict__ connect)
+{
+    const uint32_t lane = __lane_id();
+    WaveScan<K> h;
+    h.init(1e6f, lane);
+    for (uint32_t base = 0; base < N; base += 64)
+        h.step(base, base + lane < N ? sqdist(v, nodes[base + lane]) : INFINITY);
+    float dist[K];
+    uint32_t idx[K];
+    h.entries(dist, idx);
+    lomuto_sort<K>(dist, idx);
+    if (lane == 0)
+        store_scanned<K>(nodes, v, idx, r2, s, knn, spatial, connect);
+}
+
+// A surfel a lane, of those that are on; the others take nothing
+template <int K>
+__device__ __forceinline__ void scan_by_lane(const float4 *__restrict__ nodes, uint32_t N, float4 v, uint32_t s, bool on,
+                                             float r2, uint16_t *__restrict__ knn, float *__restrict__ spatial,
+                                             float *__restrict__ connect)
+{
+    ThreadScan<K> h;
+    h.init(on ? 1e6f : -1.f);
+    h.scan(0, v, nodes, N);
+    lomuto_sort<K>(h.dist, h.idx);
+    if (on)
+        store_scanned<K>(nodes, v, h.idx, r2, s, knn, spatial, connect);
+}
+
 constexpr uint32_t kSkinTile = 256;
 
 // SkinnerKernel (Skinner.cu:10-94): nodes staged through LDS in tiles.
@@ -298,21 +333,35 @@ __global__ __launch_bounds__(kSkinTile) void k_skin(const float4 *__restrict__ s
 // mostly suffice, against N distances for the scan.  Surfels that need the
 // scan (equal distances, far from all nodes) are marked in the output; when
 // a work-group has any, it puts the nodes in index order in the grid's place
-// and scans them (300k surfels, 4096 nodes, all with equal
-// distances: 1480 us, against 1500 us for the scan without the search).
+// and scans them: each wave its own, a surfel a lane, or, when they are few,
+// all waves from one list, a surfel a wave (64 candidates a step, but its sort
+// and its list's updates serve one surfel).  K = 8, 2% of the nodes there
+// twice, so a sixth of the surfels marked: 512 nodes with 20k, 100k and 300k
+// surfels 90, 140 and 220 us (each wave its own, a surfel a wave up to 24 of
+// them, 236, 277 and 397; a thread per surfel scanning all nodes, one
+// candidate after another, 164, 168 and 253).  With every distance equal to
+// some other the search comes on top of the scan (512 nodes, 300k surfels: 336
+// us, that scan 234).
 // The grid takes no memory of the caller's and none is kept between calls:
 // building it costs a work-group a few microseconds (N reads from L2), so the
 // launch is at most two 1024-thread work-groups a CU.
-// K = 8: 1.2M surfels, 4096 nodes 197 us; 300k, 1024 72 us; 20k, 256 34 us (a
-// thread per surfel scanning all nodes 2335, 370 and 99 us).
-// More than kGridNodes nodes take k_skin: 64 KB of nodes and 12 KB of cells
+// K = 8: 1.2M surfels, 4096 nodes 197 us; 300k, 1024 72 us (a thread per surfel
+// scanning all nodes, one candidate after another, 2335 and 370 us).
+// Few nodes (N K <= 512) are scanned by k_skin, equal distances or not, for
+// most need not be tied for the search to cost more; nodes spread evenly, 80
+// and 290 surfels a node, scan and grid in us: K = 4, 64 nodes 13 13 and 20 24,
+// 128 nodes 22 19 and 24 29, 192 nodes 28 26 and 26 31; K = 8, 64 nodes 22 22
+// and 25 29, 96 nodes 29 27 and 30 34, 128 nodes 36 32 and 30 36.
+// More than kGridNodes nodes take k_skin too: 64 KB of nodes and 12 KB of cells
 // leave room for two work-groups a CU, and a graph of the solver has no more.
+constexpr uint32_t kScanEntries = 512;
 constexpr uint32_t kGridNodes = 4096;
 constexpr uint32_t kGridCells = 6144; // at most, and 3/2 N (a small set's grid is cheap to build)
 constexpr uint32_t kGridThreads = 1024;
 constexpr uint32_t kGridGroups = 512; // two for each of the 256 CUs
 constexpr uint16_t kToScan = 0xffffu; // first id of a surfel that the grid leaves to the scan (no id: N <= 4096)
-constexpr uint32_t kScanLanes = 24;   // more such surfels than this in a wave: each lane scans its own
+constexpr uint32_t kFewShare = 16; // N / 16 + 16 marked surfels of a work-group are few: shared by its waves
+static_assert((kGridNodes / kFewShare + kFewShare) * 8 <= kGridCells, "their list lies in the cells' words");
 constexpr float kFarCells = 2.f;
 constexpr int kMaxShells = 6; // at most 13^3 cells, about a third of a full grid's
 
@@ -375,11 +424,12 @@ __global__ __launch_bounds__(kGridThreads, 8) void k_skin_grid(const float4 *__r
 {
     constexpr uint32_t NT = kGridThreads;
     extern __shared__ float4 gnode[]; // N nodes in cell order, w = the id's bits
-    __shared__ uint32_t cend[kGridCells / 2]; // the ends of the cells, two 16-bit counts a word
+    __shared__ __align__(16) uint32_t cend[kGridCells / 2]; // the ends of the cells, two 16-bit counts a word
     __shared__ float red[NT / 64][6];
     __shared__ uint32_t wsum[NT / 64];
     __shared__ uint32_t n_scan; // surfels left to the scan
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(tid >> 6)));
 
     // ---- bounding box (NaN coordinates leave it as it is)
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -628,49 +678,35 @@ __global__ __launch_bounds__(kGridThreads, 8) void k_skin_grid(const float4 *__r
     if (n_scan == 0)
         return;
 
-    // ---- the marked surfels: the nodes in index order in the grid's place,
-    // and each wave goes through its surfels again
-    for (uint32_t i = tid; i < N; i += NT)
+    // ---- the marked surfels: the nodes in index order in the grid's place
+    // (the lane is asked for again, so that no register keeps it till here)
+    const uint32_t ln = __lane_id();
+    for (uint32_t i = wave * 64u + ln; i < N; i += NT)
         gnode[i] = nodes[i];
+    if (wave == 0u && ln == 0u)
+        wsum[0] = 0u;
     __syncthreads();
+    const uint32_t n = n_scan;
+    const bool few = n <= N / kFewShare + kFewShare;
+    float4 *__restrict__ list = reinterpret_cast<float4 *>(cend);
     for (uint32_t chunk = chunk0; chunk < (S + 63u) / 64u; chunk += (NT / 64) * gridDim.x)
     {
-        const uint32_t s = chunk * 64u + lane;
+        const uint32_t s = chunk * 64u + ln;
         const bool to_do = s < S && knn[size_t(s) * K] == kToScan;
-        unsigned long long m = __ballot(to_do);
-        if (m == 0)
-            continue;
-        const float4 v = surfels[s < S ? s : S - 1];
-        if (uint32_t(__popcll(m)) > kScanLanes)
+        const float4 v = surfels[min(s, S - 1u)];
+        if (few)
         {
-            ThreadScan<K> h;
-            h.init(to_do ? 1e6f : -1.f); // the other lanes take nothing
-            h.scan(0, v, gnode, N);
-            lomuto_sort<K>(h.dist, h.idx);
-            if (to_do)
-                store_scanned<K>(nodes, v, h.idx, r2, s, knn, spatial, connect);
-            continue;
+            if (to_do) // listed in the cells' place
+                list[atomicAdd(&wsum[0], 1u)] = make_float4(v.x, v.y, v.z, __uint_as_float(s));
         }
-        for (; m; m &= m - 1)
-        {
-            const int l = __ffsll(m) - 1;
-            float4 q;
-            q.x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), l));
-            q.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), l));
-            q.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.z), l));
-            q.w = 0.f;
-            WaveScan<K> h;
-            h.init(1e6f);
-            for (uint32_t base = 0; base < N; base += 64)
-                h.step(base, base + lane < N ? sqdist(q, gnode[base + lane]) : INFINITY);
-            float hd[K];
-            uint32_t hx[K];
-            h.entries(hd, hx);
-            lomuto_sort<K>(hd, hx);
-            if (int(lane) == l)
-                store_scanned<K>(nodes, v, hx, r2, s, knn, spatial, connect);
-        }
+        else if (__any(to_do))
+            scan_by_lane<K>(gnode, N, v, s, to_do, r2, knn, spatial, connect);
     }
+    if (!few)
+        return;
+    __syncthreads();
+    for (uint32_t i = wave; i < n; i += NT / 64)
+        scan_by_wave<K>(gnode, N, list[i], r2, __float_as_uint(list[i].w), knn, spatial, connect);
 }
 
 // ------------------------------------------------------------ node graph
@@ -698,7 +734,7 @@ __global__ __launch_bounds__(kGraphThreads) void k_node_graph(const float4 *__re
     const uint32_t i = blockIdx.x * (kGraphThreads / 64) + (threadIdx.x >> 6);
     const float4 vi = nodes[min(i, N - 1)];
     WaveScan<K> h;
-    h.init(1e3f);
+    h.init(1e3f, lane);
     for (uint32_t base = 0; base < N; base += kGraphTile)
     {
         const uint32_t cnt = min(kGraphTile, N - base);
@@ -733,7 +769,7 @@ template <int K>
 hipError_t start_skin(const float4 *surfels, uint32_t S, const float4 *nodes, uint32_t N, float r2, uint16_t *knn,
                       float *spatial, float *connect, hipStream_t st)
 {
-    if (N > kGridNodes)
+    if (N * K <= kScanEntries || N > kGridNodes)
     {
         hipLaunchKernelGGL(k_skin<K>, dim3((S + kSkinTile - 1) / kSkinTile), dim3(kSkinTile), 0, st, surfels, S,
                            nodes, N, r2, knn, spatial, connect);

@@ -94,6 +94,25 @@ def test_skin_wide_and_long(torch_dev, S, N):
     assert np.allclose(w.cpu().numpy(), rw, rtol=2e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("kind", ["sphere", "lattice", "some_ties"])
+@pytest.mark.parametrize("S,N", [(900, 64), (900, 65), (900, 128), (900, 129), (5000, 300), (60001, 300), (300007, 300),
+                                 (200, 2000)])
+def test_skin_scan_rules(torch_dev, kind, S, N):
+    """Both sides of the limits up to which the nodes are scanned without the grid, and surfels that the grid leaves to
+    the scan: few of a work-group (a wave each), and more (a lane each)."""
+    import sho
+    from starhub_amd import native
+    torch = torch_dev
+    for K in (4, 8):
+        rng = np.random.default_rng(S + N)
+        s, n, r2 = _points(kind, S, N, rng)
+        s, n = _four(s), _four(n)
+        knn, w, _ = native.skin_surfels(torch.from_numpy(s).cuda(), torch.from_numpy(n).cuda(), K, r2)
+        rk, rw, _ = sho.skin(s, n, K, r2)
+        assert np.array_equal(knn.cpu().numpy().view(np.uint16), rk), K
+        assert np.allclose(w.cpu().numpy(), rw, rtol=2e-5, atol=1e-7), K
+
+
 def test_skin_non_finite_and_unaligned(torch_dev):
     """NaN and infinite positions take the scan's result, and outputs off a 16-byte boundary are stored as such."""
     import ctypes
