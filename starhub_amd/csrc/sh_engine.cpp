@@ -222,11 +222,9 @@ int Engine::init(const sh_solver_config &c, uint32_t max_slots)
     A(d_slots_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot));
     A(d_slots2_, size_t(max_slots) * kPcgMaxGroups * sizeof(PcgSlot2));
     A(d_flags_, 64);
-    // The resident PCG's groups wait for each other through d_slots_, and how
-    // long depends on which 4 KB page of memory that is: a solve of 200 nodes
-    // takes 806 to 866 us with only that page changed (pages two apart differ
-    // by 25 to 55 us, neighbouring pairs agree), and the allocations before it
-    // decide.  So arrays that the exchange does not use are allocated behind it.
+    // How long the resident PCG's groups wait for each other depends on the page
+    // that their slots lie in (solve_barrier_sum), and the allocations before
+    // them decide that: arrays that the exchange does not use lie behind them.
     for (Slot &sl : slots_)
     {
         SolveDesc &d = sl.d;

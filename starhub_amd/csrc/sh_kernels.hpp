@@ -169,9 +169,7 @@ hipError_t launch_rows_combine(const SolveDesc *sds, const uint32_t *row_map, in
 // once: the launch always drains, with meaningless sums.
 struct PcgSlot
 {
-    double v[2];
-    uint32_t epoch;
-    uint32_t pad[3];
+    uint64_t w[2][2]; // by the barrier number's parity: the partial's low and high half, each above the number
 };
 // Blocks of the normal matrix per persistent-PCG work-group (sets the
 // number of groups per solve, at most kPcgMaxGroups).

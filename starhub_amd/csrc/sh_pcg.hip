@@ -63,32 +63,47 @@ __device__ __forceinline__ double group_sum(double v, double *sh)
 }
 
 // Barrier of the G groups of one solve, fused with the sum of their partials.
-// Group g publishes (value, epoch) in its own slot; wave 0 of every group waits
-// for all G epochs and sums the G values in slot order, so every group gets
-// the same total, bit for bit.  Values alternate between two entries by
-// epoch parity: a group can only overwrite an entry two barriers later, after
-// every group has read it.  A wait that exceeds the spin cap sets *err and
-// ends every later wait at once, so each wave always exits.
+// Group g publishes its partial in its own slot as two words, each half of it
+// above the barrier's sequence number, behind a release fence for the vectors;
+// wave 0 of every group polls all G slots' words until they carry the number,
+// and then has the partials too: a value that is read only once an epoch word
+// has been seen is one trip to memory more, and how long a trip takes depends
+// on where the slots lie (sixteen solvers of 200 nodes made one after another,
+// so in other places, six launches of three groups each: 764 to 829 us a solve;
+// with an epoch word 795 to 865; 1024 nodes 2480 and 2590, 4096 nodes 3860 and
+// 4330).  The G values are summed in slot order, so every group gets the same
+// total, bit for bit.
+// Words alternate between two entries by the number's parity: a group can only
+// overwrite an entry two barriers later, after every group has read it, so a
+// poll meets the number before the last or the one it waits for.  A wait that
+// exceeds the spin cap sets *err and ends every later wait at once, so each
+// wave always exits.
 __device__ double solve_barrier_sum(double part, PcgSlot *__restrict__ slots, uint32_t b0, uint32_t G, uint32_t ep,
                                     uint32_t *__restrict__ err, uint32_t cap, double *sh)
 {
     if (threadIdx.x == 0)
     {
-        PcgSlot &me = slots[blockIdx.x];
-        me.v[ep & 1u] = part;
-        __hip_atomic_store(&me.epoch, ep, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t *w = slots[blockIdx.x].w[ep & 1u];
+        const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(part));
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_store(&w[0], bits << 32 | ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&w[1], (bits >> 32 << 32) | ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (threadIdx.x < 64)
     {
         double v = 0.0;
         for (uint32_t i = threadIdx.x; i < G; i += 64)
         {
-            PcgSlot &o = slots[b0 + i];
+            const uint64_t *w = slots[b0 + i].w[ep & 1u];
+            uint64_t lo, hi;
             unsigned spins = 0;
-            // relaxed polling (no cache invalidation per poll), one acquire
-            // fence once the epoch is seen
-            while (__hip_atomic_load(&o.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ep)
+            // relaxed polling: no cache invalidation per poll
+            for (;;)
             {
+                lo = __hip_atomic_load(&w[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                hi = __hip_atomic_load(&w[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (uint32_t(lo) == ep && uint32_t(hi) == ep)
+                    break;
                 __builtin_amdgcn_s_sleep(1);
                 if (++spins >= cap || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
                 {
@@ -96,9 +111,10 @@ __device__ double solve_barrier_sum(double part, PcgSlot *__restrict__ slots, ui
                     break;
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            v += __hip_atomic_load(&o.v[ep & 1u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v += __longlong_as_double(static_cast<long long>(lo >> 32 | (hi >> 32 << 32)));
         }
+        // the vectors behind the numbers seen
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1)
             v += __shfl_xor(v, o, 64);
