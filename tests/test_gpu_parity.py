@@ -587,6 +587,25 @@ def test_pipelined_pcg_many_groups_vs_fp64(torch_dev):
     say("4096-node pipelined warp error vs replayed fp64", err, "flips", flips)
 
 
+@pytest.mark.parametrize("flags,rows", [(0, 85), (0, 17), (0, 5), (8, 0)])
+def test_resident_pcg_groups_vs_fp64(torch_dev, flags, rows):
+    """The two-barrier persistent PCG with 13 groups, 65 (two rounds of slots a lane, the second of one) and 220, and
+    its streaming variant: the warp field is within the FP64 oracle's tolerance, and no wait fell back."""
+    import sho
+    from starhub_amd import native, scene, workload
+    cfg = scene.config_batch_member(1100, 978)
+    sc = scene.generate(cfg)
+    frame, prod = workload.device_frame(sc)
+    s = native.WarpSolver(native.make_config(cfg.solver, cfg.width, cfg.height, cfg.num_nodes, cfg.K, flags=flags))
+    if rows:
+        native.set_tuning(s, flags, 0, rows)
+    for _ in range(2):  # the second solve starts from the numbers the first one left
+        s.process_frame(frame)
+    assert native.pcg_fallbacks(s) == 0
+    err, _, flips = solver_check(s, workload.host_inputs(sc, prod), cfg.solver, sho.max_threads())
+    say("resident", flags, rows, "warp error vs replayed fp64", err, "flips", flips)
+
+
 def test_empty_frame_gives_identity(torch_dev):
     from starhub_amd import scene, workload
     sc = scene.generate(scene.config_c1())
